@@ -8,22 +8,112 @@
 namespace rs {
 namespace {
 
-// Elementwise move of 16-bit values between token-major rows
-// [count][kv_heads][D] (token first+t at row t) and the page layout.
-template <bool IS_V, bool TO_PAGES>
-__global__ __launch_bounds__(256)
-void convert_pages(unsigned short *pages, unsigned short *rows, int kv_heads, int D,
-                   size_t head_stride, int first, size_t total) {
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (size_t)gridDim.x * blockDim.x) {
-        const int d = (int)(e % D);
-        const size_t th = e / D;
-        const int h = (int)(th % kv_heads);
-        const int token = first + (int)(th / kv_heads);
-        const size_t off = (size_t)h * head_stride +
-                           (IS_V ? v_page_offset(token, d, D) : k_page_offset(token, d, D));
-        if (TO_PAGES) pages[off] = rows[e];
-        else rows[e] = pages[off];
+// Token-major rows [count][kv_heads][D] (token first+t at row t) <-> pages.
+// A block moves one (page, KV head) of K or of V, K's and V's blocks in one
+// launch, KV heads fastest, so that neighbouring blocks share the 32 rows'
+// lines.  The move is bound by HBM (read once, written once), so every thread
+// moves 16-byte pieces of the pages:
+//   K: a piece is 8 dims of one token on both sides.  Pages are accessed
+//      contiguously, rows in 64-byte parts of 16 rows per wave instruction.
+//   V: a piece is 8 tokens of one dim, so a thread takes VD dims of the 8
+//      tokens of one key group (8 row accesses of 4 or 8 bytes, a wave
+//      covering whole row parts) and transposes them in registers.
+// Only tokens first .. first+count-1 are touched: other tokens' rows do not
+// exist, and their page slots keep their values (a V piece that holds such a
+// token is written value by value).  Buffers that are not 16-byte aligned
+// move value by value throughout.
+// Rows taken into pages are loaded non-temporally (each is read once: 39.5 ->
+// 36.7 us); pages are loaded with the default policy (straight after their
+// writes they are partly cached: 29.1 against 40.4 us non-temporally).
+// 20,001 tokens of 4 x 256 dims (82 MB read and written each way), rocprof
+// medians: 36.7 us into pages and 29.1 us back, 4.5 and 5.6 TB/s of read +
+// write; four launches that moved value by value took 45-60 us each (207 us).
+struct ConvertArgs {
+    unsigned short *pages[2], *rows[2];   // K, V (both NULL on a side that is not moved)
+    size_t head_stride;
+    int kv_heads, first, count, page0, n_pages;
+    bool whole;                           // 16-byte aligned buffers
+};
+constexpr int kConvertThreads = 256;
+
+template <int D, bool TO_PAGES>
+__global__ __launch_bounds__(kConvertThreads)
+void convert_pages(ConvertArgs a) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int PAGE = 32 * D;
+    const int sides = (a.pages[0] ? 1 : 0) + (a.pages[1] ? 1 : 0);
+    const size_t blocks = (size_t)a.n_pages * a.kv_heads * sides;
+    const size_t row_stride = (size_t)a.kv_heads * D;
+    for (size_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const int h = (int)(b % a.kv_heads);
+        const size_t ps = b / a.kv_heads;
+        const int side = sides == 2 ? (int)(ps % 2) : a.pages[0] ? 0 : 1;
+        const int page = a.page0 + (int)(sides == 2 ? ps / 2 : ps);
+        unsigned short *pg = a.pages[side] + (size_t)h * a.head_stride + (size_t)page * PAGE;
+        // Row of the page's token p: rows + p * row_stride (signed: the first
+        // page may start before `first`).
+        unsigned short *rows = a.rows[side] + ((long long)page * 32 - a.first) * (long long)row_stride + (size_t)h * D;
+        const int lo = max(a.first - page * 32, 0);                          // valid tokens of the page: lo .. hi-1
+        const int hi = (int)min((long long)a.first + a.count - (long long)page * 32, 32LL);
+        if (!a.whole || (TO_PAGES && side == 1 && hi - lo < 32)) {
+            for (int e = lo * D + threadIdx.x; e < hi * D; e += kConvertThreads) {
+                const int p = e / D, d = e % D;
+                const size_t off = side ? v_page_offset(p, d, D) : k_page_offset(p, d, D);
+                if (TO_PAGES) pg[off] = rows[p * row_stride + d];
+                else rows[p * row_stride + d] = pg[off];
+            }
+        } else if (side == 0) {
+            constexpr int PER = PAGE / 8 / kConvertThreads;
+            u32x4 v[PER];
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int c = threadIdx.x + i * kConvertThreads;   // piece of the page
+                const int p = c / (2 * D) * 16 + c % 16, d = c / 16 % (D / 8) * 8;
+                if (p < lo || p >= hi) continue;
+                v[i] = TO_PAGES ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(rows + p * row_stride + d))
+                                : *reinterpret_cast<const u32x4 *>(pg + c * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int c = threadIdx.x + i * kConvertThreads;
+                const int p = c / (2 * D) * 16 + c % 16, d = c / 16 % (D / 8) * 8;
+                if (p < lo || p >= hi) continue;
+                if (TO_PAGES) *reinterpret_cast<u32x4 *>(pg + c * 8) = v[i];
+                else *reinterpret_cast<u32x4 *>(rows + p * row_stride + d) = v[i];
+            }
+        } else {
+            constexpr int VD = PAGE / 8 / kConvertThreads;   // dims per thread (4 or 2): D / VD threads per key group
+            typedef unsigned short VP __attribute__((ext_vector_type(VD)));
+            typedef unsigned short V8 __attribute__((ext_vector_type(8)));
+            const int g = threadIdx.x / (D / VD), d = threadIdx.x % (D / VD) * VD;
+            unsigned short *slots = pg + d / 16 * 512 + g * 128 + d % 16 * 8;
+            VP x[8];
+            V8 s[VD];
+            if constexpr (!TO_PAGES) {
+#pragma unroll
+                for (int k = 0; k < VD; ++k) s[k] = *reinterpret_cast<const V8 *>(slots + k * 8);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int p = j / 4 * 16 + g * 4 + j % 4;   // slot j's token
+                VP *row = reinterpret_cast<VP *>(rows + p * row_stride + d);
+                if constexpr (TO_PAGES) {
+                    x[j] = __builtin_nontemporal_load(row);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < VD; ++k) x[j][k] = s[k][j];
+                    if (p >= lo && p < hi) *row = x[j];
+                }
+            }
+            if constexpr (TO_PAGES) {
+#pragma unroll
+                for (int k = 0; k < VD; ++k) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) s[k][j] = x[j][k];
+                    *reinterpret_cast<V8 *>(slots + k * 8) = s[k];
+                }
+            }
+        }
     }
 }
 
@@ -31,24 +121,30 @@ template <bool TO_PAGES>
 void convert(void *k_pages, void *v_pages, const void *k_rows, const void *v_rows,
              int kv_heads, int head_dim, int capacity, int first, int count,
              hipStream_t stream) {
-    const size_t total = (size_t)count * kv_heads * head_dim;
-    if (!total) return;
-    const size_t stride = (size_t)capacity * head_dim;
-    const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 65536);
-    if (k_pages && k_rows) {
-        hipLaunchKernelGGL((convert_pages<false, TO_PAGES>), dim3(blocks), dim3(256), 0, stream,
-                           static_cast<unsigned short *>(k_pages),
-                           const_cast<unsigned short *>(static_cast<const unsigned short *>(k_rows)),
-                           kv_heads, head_dim, stride, first, total);
-        check(hipGetLastError());
-    }
-    if (v_pages && v_rows) {
-        hipLaunchKernelGGL((convert_pages<true, TO_PAGES>), dim3(blocks), dim3(256), 0, stream,
-                           static_cast<unsigned short *>(v_pages),
-                           const_cast<unsigned short *>(static_cast<const unsigned short *>(v_rows)),
-                           kv_heads, head_dim, stride, first, total);
-        check(hipGetLastError());
-    }
+    if (!count) return;
+    ConvertArgs a = {};
+    auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    a.whole = true;
+    auto add = [&](int side, void *pages, const void *rows) {
+        if (!pages || !rows) return;
+        a.pages[side] = static_cast<unsigned short *>(pages);
+        a.rows[side] = const_cast<unsigned short *>(static_cast<const unsigned short *>(rows));
+        a.whole = a.whole && aligned(pages) && aligned(rows);
+    };
+    add(0, k_pages, k_rows);
+    add(1, v_pages, v_rows);
+    a.head_stride = (size_t)capacity * head_dim;
+    a.kv_heads = kv_heads;
+    a.first = first;
+    a.count = count;
+    a.page0 = first / kPageTokens;
+    a.n_pages = (int)(((long long)first + count + kPageTokens - 1) / kPageTokens) - a.page0;
+    const size_t blocks = (size_t)a.n_pages * kv_heads * ((a.pages[0] != nullptr) + (a.pages[1] != nullptr));
+    const void *kernel = head_dim == 256 ? (const void *)&convert_pages<256, TO_PAGES>
+                                         : (const void *)&convert_pages<128, TO_PAGES>;
+    void *args[] = {&a};
+    check(hipLaunchKernel(kernel, dim3((unsigned)std::min<size_t>(blocks, 1u << 20)), dim3(kConvertThreads), args, 0,
+                          stream));
 }
 
 // One wave per (head, token): heads 0..23 are query heads, 24..27 the KV
