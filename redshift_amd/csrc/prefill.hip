@@ -4,7 +4,8 @@
 // qvelox/server.py:187-191); this is the same causal GQA formula for long
 // token runs: row t sees keys 0..position+t.
 //
-// One workgroup owns 192 query rows of one KV head (row = token * group +
+// One workgroup owns 192 query rows (128 at head_dim 128, two tiles per wave:
+// kPairRows) of one KV head (row = token * group +
 // query head within the group) as twelve 16-row tiles, one per wave (three
 // per SIMD), whose query fragments stay in registers.  The tiles are dealt
 // out so that every SIMD has about the same number of (row, key) pairs (see
@@ -176,45 +177,55 @@ __device__ __forceinline__ int v_slot_token(int g, int j) {
 // so the same bits) and its workgroup 0 appends them to the pages.  No
 // workgroup reads a key that another one appends.  (kPrepQuery: qn_stage is
 // 1 KiB of LDS per wave, for the q_norm weights.)
+// NT: 16-row tiles per wave (adjacent rows); their scores and outputs share
+// every K and V fragment read from LDS.
+// KG: wave groups that share the rows, each taking every KG-th page; their
+// states are merged through the rings (and `merge_ml`, 1 KiB of LDS per row
+// wave) at the end.
 template <int D, typename KV, typename VT, bool PSPLIT, bool QSPLIT, int MODE, int ROWS, int PASS = -1,
-          int PREP = 0>
+          int PREP = 0, int NT = 1, int KG = 1>
 __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT *vring, const void *v_pages,
-                                             size_t v_head_stride, float *qn_stage = nullptr) {
+                                             size_t v_head_stride, float *qn_stage = nullptr,
+                                             float *merge_ml = nullptr) {
     using V8 = typename Vec8<KV>::type;
     using OUT = std::conditional_t<MODE == kOutSame, KV, float>;
     typedef uint32_t U4 __attribute__((ext_vector_type(4)));
     using PT = VT;
     using PV8 = typename Vec8<PT>::type;
-    constexpr int kPWaves = PASS < 0 ? ROWS / 16 : 8;
+    constexpr int TR = 16 * NT;                        // rows per wave
+    constexpr int kPWaves = PASS < 0 ? ROWS / TR * KG : 8;
     static_assert(PASS < 0 || ROWS == 3 * 4 * 16, "two passes of eight waves over three rounds of tiles");
     constexpr bool PQ = (PREP & kPrepQuery) != 0, PK = (PREP & kPrepKeys) != 0;
     static_assert(!PQ || (D == kModelHeadDim && QSPLIT && PSPLIT && MODE == kOutGated &&
                           std::is_same<KV, _Float16>::value && std::is_same<VT, _Float16>::value),
                   "the prepared query is the fused model's: fp32 query as hi + lo parts, gated output");
     static_assert(!PK || (PQ && PASS < 0), "the chunk's own keys come with its prepared query, in one pass");
+    static_assert(NT == 1 || (PREP == 0 && PASS < 0), "several tiles per wave: the raw instances");
+    static_assert(KG == 1 || (NT == 2 && KG == 2 && kPWaves == 8 && D == 128), "two groups of four waves");
     constexpr int KS = D / 32, DT = D / 16;
     constexpr int PAGE = 32 * D;                       // elements of one K (or V) page
     constexpr int PAGE_BYTES = PAGE * 2;
     // The first kLoaders waves (two per SIMD of twelve, one per SIMD of
     // eight) copy the pages, H 1 KiB loads each per K (or V) page.
-    constexpr int kLoaders = kPWaves == 12 ? 8 : kPWaves / 2;
+    constexpr int kLoaders = kPWaves == 12 ? 8 : NT == 2 ? kPWaves : kPWaves / 2;
     constexpr int H = PAGE_BYTES / 1024 / kLoaders;
     static_assert(H >= 1 && PAGE_BYTES / 1024 % kLoaders == 0, "loads divide over the loader waves");
 
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave index (uniform)
     const int h = blockIdx.x % a.kv_heads;
-    // Load balance.  The R rows of a KV head form T = ceil(R/16) tiles of 16
-    // rows; a later tile sees more keys.  Wave w of workgroup j runs on SIMD
-    // w % 4 and serves slot k = 4j + w%4 (K = 4 n_tiles slots per head) in
-    // round w / 4, which deals the tiles out serpentine-wise:
+    // Load balance.  The R rows of a KV head form T = ceil(R/TR) tiles of TR
+    // rows (TR = 16 NT); a later tile sees more keys.  Wave w of workgroup j
+    // runs on SIMD w % 4 and serves slot k = 4j + w%4 (K = 4 n_tiles slots per
+    // head) in round w / 4, which deals the tiles out serpentine-wise:
     //   round 0: tile T-1-k    (the last K tiles, the latest first)
     //   round 1: tile T-2K+k   (the K before them, in rising order)
     //   round 2: tile T-3K+k   (the rest, rising)
     // Rounds 0 and 1 give every slot the same key count; round 2 rises with
     // k, while the stretch in which only the round-0 wave still has pages
-    // shrinks with k.  So every SIMD, and every workgroup, has about the
-    // same work.  Negative tiles are padding, and rows from R on are not
+    // shrinks with k.  So every SIMD, and every workgroup, has about the same
+    // work.  (One round, NT = 2: the workgroups start with the longest, and
+    // those that follow fill the CUs as they end.)  Negative tiles are padding, and rows from R on are not
     // stored.  Workgroup j's last row lies in its round-0 tile of slot 4j.
     const int R = a.rows;
     const int rest = blockIdx.x / a.kv_heads;
@@ -222,11 +233,12 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // kPrepKeys: the last run attends to the chunk's keys too (uniform per workgroup).
     const bool new_keys = PK && split == a.splits - 1;
     static_assert(kPWaves % 4 == 0 && kPWaves / 4 <= 3, "one to three rounds of four waves");
-    const int T = (R + 15) / 16, K = 4 * a.n_tiles, slot = 4 * j + (w & 3);
-    const int round = PASS == 1 ? (w < 4 ? 2 : 3) : w >> 2;   // round 3: no tile
+    const int T = (R + TR - 1) / TR, K = 4 * a.n_tiles, slot = 4 * j + (w & 3);
+    const int kg = KG == 1 ? 0 : w >> 2;                      // this wave's pages: kg, kg + KG, ...
+    const int round = PASS == 1 ? (w < 4 ? 2 : 3) : KG == 1 ? w >> 2 : 0;   // round 3: no tile
     const int tile = round == 0 ? T - 1 - slot : round == 1 ? T - 2 * K + slot
                    : round == 2 ? T - 3 * K + slot : -1;
-    const int row0 = 16 * tile;
+    const int row0 = TR * tile;
     const int row_end = R;                                              // valid rows: [0, row_end)
 
     // Query fragments (B operand): k-step ks of lane l holds row row0 + l%16,
@@ -237,8 +249,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // the first K page covers its query, and the other waves wait for their
     // query alone.  (As compiler-tracked loads, the compiler would wait for
     // every page in flight before their first use.)
-    V8 qf[KS], qlo[QSPLIT ? KS : 1];
-    int limit;
+    V8 qf[NT][KS], qlo[QSPLIT ? KS : 1];
+    static_assert(NT == 1 || !QSPLIT, "a precise query takes one tile per wave");
+    int limit[NT];
     [[maybe_unused]] int row_token;
     // kPrepQuery: the row's fp32 query in the same layout (k-step ks: two float4),
     // and the q_norm weights as the prepare kernel holds them (lane l: dims
@@ -249,12 +262,13 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // prep_query), evaluated while the query loads are in flight.
     [[maybe_unused]] float ca = 0.f, sa = 0.f, cb = 0.f, sb = 0.f;
     [[maybe_unused]] int qpos = 0, tile_pos = 0;
-    {
-        const int row = min(max(row0 + (lane & 15), 0), max(row_end, 1) - 1);
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+        const int row = min(max(row0 + 16 * tt + (lane & 15), 0), max(row_end, 1) - 1);
         const int t = row / a.group, gg = row - t * a.group;
         // kPrepKeys' cached runs: every row sees every cached key.
         row_token = t;
-        limit = PK ? a.position - 1 : a.position + t;
+        limit[tt] = PK ? a.position - 1 : a.position + t;
         if constexpr (PQ) {
             qpos = a.position + t;
             // The position of the tile's first (clamped) row's token; the
@@ -272,7 +286,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             const KV *src = static_cast<const KV *>(a.q) +
                             ((size_t)t * a.q_heads + (size_t)h * a.group + gg) * D + 8 * g;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) global_load16(qf[ks], src + 32 * ks);
+            for (int ks = 0; ks < KS; ++ks) global_load16(qf[tt][ks], src + 32 * ks);
             if constexpr (QSPLIT) {
                 const KV *lo = static_cast<const KV *>(a.q_lo) + (src - static_cast<const KV *>(a.q));
 #pragma unroll
@@ -285,7 +299,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // T-3K+4j+3; none when that tile is padding).
     // (kPrepKeys: the cached keys 0 .. position-1 first.)
     const int last_tile = PASS == 1 ? T - 3 * K + 4 * j + 3 : T - 1 - 4 * j;
-    const int wg_keys = last_tile < 0 ? 0 : a.position + (min(16 * (last_tile + 1), R) - 1) / a.group + 1;
+    const int wg_keys = last_tile < 0 ? 0 : a.position + (min(TR * (last_tile + 1), R) - 1) / a.group + 1;
     int n_keys = PK && last_tile >= 0 ? a.position : wg_keys;
     const int n = (n_keys + 31) / 32;
     // This split's pages: p0 + i for i = 0 .. nl-1 (local index i, ring
@@ -295,7 +309,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     int p0 = split * sp;
     int nl = max(0, min(n, p0 + sp) - p0);
     // Pages of this wave: those its last valid row sees (none without one).
-    const int wave_last = min(row0 + 15, row_end - 1);
+    const int wave_last = min(row0 + TR - 1, row_end - 1);
     const int wave_keys = wave_last < max(row0, 0) ? 0 : a.position + wave_last / a.group + 1;
     int nw = min(max((PK && wave_keys ? n : (wave_keys + 31) / 32) - p0, 0), nl);
     // Pages from which on some row of this wave masks keys (every row sees
@@ -304,6 +318,13 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // chunk keys: the cached ones of their first page).
     int wave_first_limit = PK ? a.position - 1 : a.position + max(row0, 0) / a.group;
     int key_lo = 0;
+    if constexpr (NT == 2) {
+        // The wave's last step runs one softmax past its last page.
+        const int end = (p0 + nw) * 32 - 1;
+        wave_first_limit = min(wave_first_limit, end);
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) limit[tt] = min(limit[tt], end);
+    }
     // kPrepKeys: pages come from the LDS rings as the workgroup prepared them
     // (the chunk's keys) rather than from global memory.
     [[maybe_unused]] bool from_lds = false;
@@ -325,24 +346,31 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     const uint32_t kring_lane = lds_addr(kring) + lane * 16;
     const uint32_t vring_lane = lds_addr(vring) + lane * 16;
 
-    f32x4 acc[DT];
+    f32x4 acc[NT][DT];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[tt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // m stays -inf for a row that sees no key of its pages (a split past its
     // last key).  Its exponents are taken against 0 instead (mu below), so
     // they are exp2(-inf) = 0 and the row's sum and accumulators stay 0: no
     // operation of this file makes a NaN, which matters because it is
     // compiled with -fno-honor-nans.  Such a row's partial is stored as
     // empty.
-    float m = -INFINITY, l = 0.f;
+    float m[NT], l[NT];
     // The scores are scaled by a positive factor in the exponents; a negative
     // or zero scale's sign is applied to the scores themselves.  A row's max
     // moves past move_above = (unscaled max) + kLazy / scale.
     const float sign = a.scale_log2 > 0.f ? 1.f : a.scale_log2 < 0.f ? -1.f : 0.f;
     const float scale = a.scale_log2 == 0.f ? 1.f : __builtin_fabsf(a.scale_log2);
     const float lazy = kLazy / scale;
-    float move_above = -INFINITY, neg_mu = 0.f;
-    f32x4 s[2];            // scores of the page whose softmax comes next
+    float move_above[NT], neg_mu[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+        m[tt] = move_above[tt] = -INFINITY;
+        l[tt] = neg_mu[tt] = 0.f;
+    }
+    f32x4 s[NT][2];        // scores of the page whose softmax comes next
 
     // ---- S^T of one page, chunk by chunk ----
     // K fragments stream through a window of KW k-steps (2 KW reads in
@@ -360,140 +388,225 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             lds_read<(16 * D + ks * 512) * 2>(kf[ks][1], kb);
         }
     };
-    auto qk_chunk = [&](auto ks_, uint32_t kb, f32x4 *sn) __attribute__((always_inline)) {
+    auto qk_chunk = [&](auto ks_, uint32_t kb, f32x4 (&sn)[NT][2]) __attribute__((always_inline)) {
         constexpr int ks = decltype(ks_)::value;
         if constexpr (ks < KS) {
             constexpr int later = 2 * (KW - 1 < KS - 1 - ks ? KW - 1 : KS - 1 - ks);
             lds_wait<later>(kf[ks][0], kf[ks][1]);
             read_k(std::integral_constant<int, ks + KW>{}, kb);
-            sn[0] = mfma(kf[ks][0], qf[ks], sn[0]);
-            sn[1] = mfma(kf[ks][1], qf[ks], sn[1]);
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) {
+                sn[tt][0] = mfma(kf[ks][0], qf[tt][ks], sn[tt][0]);
+                sn[tt][1] = mfma(kf[ks][1], qf[tt][ks], sn[tt][1]);
+            }
             if constexpr (QSPLIT) {
-                sn[0] = mfma(kf[ks][0], qlo[ks], sn[0]);
-                sn[1] = mfma(kf[ks][1], qlo[ks], sn[1]);
+                sn[0][0] = mfma(kf[ks][0], qlo[ks], sn[0][0]);
+                sn[0][1] = mfma(kf[ks][1], qlo[ks], sn[0][1]);
             }
         }
+    };
+
+    // ---- softmax of tile tt's scores of page p0 + i, in seven parts ----
+    // Each part is a few vector instructions for the step to put beside its
+    // matrix products: 0 the scores and their lane's max, 1 a moved row max,
+    // 2 and 3 the exponents, 4 and 5 P^T as B operands, 6 the row sum.
+    float x[8], e[8], mx;
+    uint32_t ph[NT][4], pl[NT][4];
+    auto softmax = [&](auto t_, auto part_, int i) __attribute__((always_inline)) {
+        constexpr int tt = decltype(t_)::value, part = decltype(part_)::value;
+        if constexpr (part == 0) {
+            // Unscaled scores; keys past a row's limit are masked.
+            const int key0 = (p0 + i) * 32;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = s[tt][j >> 2][j & 3];
+            if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo) || sign != 1.f) {
+                keep_branch();
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int key = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
+                    x[j] *= sign;
+                    if (key > limit[tt] || (PK && key < key_lo)) x[j] = -INFINITY;
+                }
+            }
+            mx = __builtin_fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], x[5]));
+            mx = max3(mx, x[6], x[7]);
+            pin(mx);
+        } else if constexpr (part == 1) {
+            // A page moves a row's max when one of its scores exceeds it by
+            // more than kLazy (or is the row's first), which any lane sees
+            // from its own keys; only then the row max over the four lane
+            // groups, the rescaling factor and the rescaled sums are worked
+            // out.  A row that sees a key of this split sees its first one on
+            // the split's first page, where its max becomes finite.
+            if (__any(mx > move_above[tt])) {
+                keep_branch();
+                mx = row_group_max(mx);
+                const bool moved = mx > move_above[tt];
+                // `moved` implies a finite mx, so m - mx * scale is never
+                // -inf - (-inf).
+                const float to = mx * scale, alpha = moved ? __builtin_amdgcn_exp2f(m[tt] - to) : 1.f;
+                m[tt] = moved ? to : m[tt];
+                move_above[tt] = moved ? mx + lazy : move_above[tt];
+                // The exponents' reference point: m, or 0 while the row has
+                // seen no key (all its scores are then -inf, and their
+                // exponents 0).
+                neg_mu[tt] = m[tt] == -INFINITY ? 0.f : -m[tt];
+                l[tt] *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) acc[tt][dt] *= alpha;
+            }
+            pin(neg_mu[tt]);
+        } else if constexpr (part <= 3) {
+            constexpr int J = 4 * (part - 2);
+#pragma unroll
+            for (int j = J; j < J + 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], scale, neg_mu[tt]));
+            pin(e[J], e[J + 1], e[J + 2], e[J + 3]);
+        } else if constexpr (part <= 5) {
+            constexpr int J = 4 * (part - 4);
+#pragma unroll
+            for (int j = J; j < J + 4; j += 2) {
+                ph[tt][j / 2] = pack2(e[j], e[j + 1], PT{});
+                if constexpr (PSPLIT)
+                    pl[tt][j / 2] = pack2(e[j] - unpack_lo(ph[tt][j / 2], PT{}),
+                                          e[j + 1] - unpack_hi(ph[tt][j / 2], PT{}), PT{});
+            }
+            pin(ph[tt][J / 2], ph[tt][J / 2 + 1]);
+            if constexpr (PSPLIT) pin(pl[tt][J / 2], pl[tt][J / 2 + 1]);
+        } else {
+            l[tt] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+            pin(l[tt]);
+        }
+    };
+    auto p_operand = [&](const uint32_t (&w4)[4]) __attribute__((always_inline)) {
+        return __builtin_bit_cast(PV8, U4{w4[0], w4[1], w4[2], w4[3]});
     };
 
     // ---- one pipeline step: S^T of page i+1, softmax and P.V of page i ----
     // (On a workgroup's last step the scores of the page after the last are
     // computed from a stale buffer and dropped.)
-    auto step = [&](int i) __attribute__((always_inline)) {
-        const uint32_t kb = kring_lane + ((i + 1) & 3) * PAGE_BYTES;
-        const uint32_t vb = vring_lane + (i & 3) * PAGE_BYTES;
-        f32x4 sn[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-        // The S^T and softmax phase runs at raised wave priority, the P.V
-        // products at the default one.  The three waves of a SIMD leave each
-        // barrier in step; with the priorities the issue arbiter lets one of
-        // them run ahead through its phase while another's V products fill
-        // the matrix pipe (2048-token chunk: 461-469 -> 447-453 us per layer).
-        __builtin_amdgcn_s_setprio(1);
-        static_for<0, KW>([&](auto ks) { read_k(ks, kb); });
-        // Scores of page p0 + i, unscaled; keys past a row's limit are masked.
-        const int key0 = (p0 + i) * 32;
-        float x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = s[j >> 2][j & 3];
-        if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo) || sign != 1.f) {
-            keep_branch();
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int key = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
-                x[j] *= sign;
-                if (key > limit || (PK && key < key_lo)) x[j] = -INFINITY;
-            }
-        }
-        float mx = __builtin_fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], x[5]));
-        mx = max3(mx, x[6], x[7]);
-        pin(mx);
-        qk_chunk(std::integral_constant<int, 0>{}, kb, sn);
-        // A page moves a row's max when one of its scores exceeds it by more
-        // than kLazy (or is the row's first), which any lane sees from its
-        // own keys; only then the row max over the four lane groups, the
-        // rescaling factor and the rescaled sums are worked out.  A row that
-        // sees a key of this split sees its first one on the split's first
-        // page, where its max becomes finite.
-        if (__any(mx > move_above)) {
-            keep_branch();
-            mx = row_group_max(mx);
-            const bool moved = mx > move_above;
-            // `moved` implies a finite mx, so m - mx * scale is never -inf - (-inf).
-            const float to = mx * scale, alpha = moved ? __builtin_amdgcn_exp2f(m - to) : 1.f;
-            m = moved ? to : m;
-            move_above = moved ? mx + lazy : move_above;
-            // The exponents' reference point: m, or 0 while the row has seen
-            // no key (all its scores are then -inf, and their exponents 0).
-            neg_mu = m == -INFINITY ? 0.f : -m;
-            l *= alpha;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
-        }
-        qk_chunk(std::integral_constant<int, 1>{}, kb, sn);
-        float e[8];
-        pin(neg_mu);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], scale, neg_mu));
-        pin(e[0], e[1], e[2], e[3]);
-        qk_chunk(std::integral_constant<int, 2>{}, kb, sn);
-#pragma unroll
-        for (int j = 4; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[j], scale, neg_mu));
-        pin(e[4], e[5], e[6], e[7]);
-        qk_chunk(std::integral_constant<int, 3>{}, kb, sn);
-        // P^T as B operands: hi parts (and lo parts, bf16).
-        uint32_t ph[4], pl[4] = {};
-#pragma unroll
-        for (int j = 0; j < 4; j += 2) {
-            ph[j / 2] = pack2(e[j], e[j + 1], PT{});
-            if constexpr (PSPLIT) {
-                pl[j / 2] = pack2(e[j] - unpack_lo(ph[j / 2], PT{}), e[j + 1] - unpack_hi(ph[j / 2], PT{}), PT{});
-            }
-        }
-        pin(ph[0], ph[1]);
-        if constexpr (PSPLIT) pin(pl[0], pl[1]);
-        qk_chunk(std::integral_constant<int, 4>{}, kb, sn);
-#pragma unroll
-        for (int j = 4; j < 8; j += 2) {
-            ph[j / 2] = pack2(e[j], e[j + 1], PT{});
-            if constexpr (PSPLIT) {
-                pl[j / 2] = pack2(e[j] - unpack_lo(ph[j / 2], PT{}), e[j + 1] - unpack_hi(ph[j / 2], PT{}), PT{});
-            }
-        }
-        pin(ph[2], ph[3]);
-        if constexpr (PSPLIT) pin(pl[2], pl[3]);
-        qk_chunk(std::integral_constant<int, 5>{}, kb, sn);
-        l += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-        pin(l);
-        static_for<6, KS>([&](auto ks) { qk_chunk(ks, kb, sn); });
-        const PV8 p_hi = __builtin_bit_cast(PV8, U4{ph[0], ph[1], ph[2], ph[3]});
-        const PV8 p_lo = __builtin_bit_cast(PV8, U4{pl[0], pl[1], pl[2], pl[3]});
+    auto step_one = [&](int i) __attribute__((always_inline)) {
+        if constexpr (NT == 1) {
+            const uint32_t kb = kring_lane + ((i + 1) & 3) * PAGE_BYTES;
+            const uint32_t vb = vring_lane + (i & 3) * PAGE_BYTES;
+            f32x4 sn[1][2] = {{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}};
+            // The S^T and softmax phase runs at raised wave priority, the P.V
+            // products at the default one.  The three waves of a SIMD leave each
+            // barrier in step; with the priorities the issue arbiter lets one of
+            // them run ahead through its phase while another's V products fill
+            // the matrix pipe (2048-token chunk: 461-469 -> 447-453 us per layer).
+            __builtin_amdgcn_s_setprio(1);
+            static_for<0, KW>([&](auto ks) { read_k(ks, kb); });
+            static_for<0, 7>([&](auto part) {
+                constexpr int P = decltype(part)::value;
+                softmax(std::integral_constant<int, 0>{}, part, i);
+                static_for<P, P == 6 ? KS : P + 1>([&](auto ks) { qk_chunk(ks, kb, sn); });
+            });
+            const PV8 p_hi = p_operand(ph[0]);
+            [[maybe_unused]] PV8 p_lo;
+            if constexpr (PSPLIT) p_lo = p_operand(pl[0]);
 
-        // ---- O^T += V^T P^T for page i ----
-        // V fragments stream through a window of VW reads.
-        constexpr int VW = 4;
-        PV8 vf[DT];
-        auto read_v = [&](auto dt_) __attribute__((always_inline)) {
-            constexpr int dt = decltype(dt_)::value;
-            if constexpr (dt < DT) lds_read<dt * 1024>(vf[dt], vb);
-        };
-        static_for<0, VW>(read_v);
-        // Pairs of tiles: the hi and lo products of a tile accumulate into
-        // the same registers, so they are issued two apart.
-        __builtin_amdgcn_s_setprio(0);
-        static_for<0, DT / 2>([&](auto dp_) {
-            constexpr int dt = 2 * decltype(dp_)::value;
-            constexpr int later = dt + 2 + VW <= DT + 2 ? VW - 2 : DT - 2 - dt;
-            lds_wait<later>(vf[dt], vf[dt + 1]);
-            read_v(std::integral_constant<int, dt + VW>{});
-            read_v(std::integral_constant<int, dt + VW + 1>{});
-            acc[dt] = mfma(vf[dt], p_hi, acc[dt]);
-            acc[dt + 1] = mfma(vf[dt + 1], p_hi, acc[dt + 1]);
-            if constexpr (PSPLIT) {
-                acc[dt] = mfma(vf[dt], p_lo, acc[dt]);
-                acc[dt + 1] = mfma(vf[dt + 1], p_lo, acc[dt + 1]);
-            }
-        });
-        s[0] = sn[0];
-        s[1] = sn[1];
+            // ---- O^T += V^T P^T for page i ----
+            // V fragments stream through a window of VW reads.
+            constexpr int VW = 4;
+            PV8 vf[DT];
+            auto read_v = [&](auto dt_) __attribute__((always_inline)) {
+                constexpr int dt = decltype(dt_)::value;
+                if constexpr (dt < DT) lds_read<dt * 1024>(vf[dt], vb);
+            };
+            static_for<0, VW>(read_v);
+            // Pairs of tiles: the hi and lo products of a tile accumulate into
+            // the same registers, so they are issued two apart.
+            __builtin_amdgcn_s_setprio(0);
+            static_for<0, DT / 2>([&](auto dp_) {
+                constexpr int dt = 2 * decltype(dp_)::value;
+                constexpr int later = dt + 2 + VW <= DT + 2 ? VW - 2 : DT - 2 - dt;
+                lds_wait<later>(vf[dt], vf[dt + 1]);
+                read_v(std::integral_constant<int, dt + VW>{});
+                read_v(std::integral_constant<int, dt + VW + 1>{});
+                acc[0][dt] = mfma(vf[dt], p_hi, acc[0][dt]);
+                acc[0][dt + 1] = mfma(vf[dt + 1], p_hi, acc[0][dt + 1]);
+                if constexpr (PSPLIT) {
+                    acc[0][dt] = mfma(vf[dt], p_lo, acc[0][dt]);
+                    acc[0][dt + 1] = mfma(vf[dt + 1], p_lo, acc[0][dt + 1]);
+                }
+            });
+            s[0][0] = sn[0][0];
+            s[0][1] = sn[0][1];
+        }
+    };
+
+    // ---- the same with two tiles per wave, half a step apart ----
+    // Tile 0's softmax of page i is done when step i begins.  Its first half
+    // runs tile 1's softmax of page i beside tile 0's products (S^T of page
+    // i+1, P.V of page i), its second half tile 0's softmax of page i+1
+    // beside tile 1's products of the same two pages, whose K and V fragments
+    // stay in registers from the first half.  So each half has as many vector
+    // as matrix cycles, from one wave, and every fragment is read from LDS
+    // once for 32 rows.  (The page after the last masks every key, so that
+    // its softmax changes nothing.)
+    auto step_two = [&](int i) __attribute__((always_inline)) {
+        if constexpr (NT == 2) {
+            const uint32_t kb = kring_lane + ((i + KG) & 3) * PAGE_BYTES;
+            const uint32_t vb = vring_lane + (i & 3) * PAGE_BYTES;
+            constexpr std::integral_constant<int, 0> t0{};
+            constexpr std::integral_constant<int, 1> t1{};
+            static_assert(KS == 4 && DT == 8, "all fragments of a page in flight or in registers");
+            PV8 vf[DT];
+            auto read_v = [&](auto dt_) __attribute__((always_inline)) {
+                constexpr int dt = decltype(dt_)::value;
+                if constexpr (dt < DT) lds_read<dt * 1024>(vf[dt], vb);
+            };
+            auto pv = [&](auto t_, auto dt_, PV8 hi, PV8 lo) __attribute__((always_inline)) {
+                constexpr int tt = decltype(t_)::value, dt = decltype(dt_)::value;
+                acc[tt][dt] = mfma(vf[dt], hi, acc[tt][dt]);
+                if constexpr (PSPLIT) acc[tt][dt] = mfma(vf[dt], lo, acc[tt][dt]);
+            };
+            auto qk = [&](auto t_, auto ks_) __attribute__((always_inline)) {
+                constexpr int tt = decltype(t_)::value, ks = decltype(ks_)::value;
+                if constexpr (ks == 0) s[tt][0] = s[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                s[tt][0] = mfma(kf[ks][0], qf[tt][ks], s[tt][0]);
+                s[tt][1] = mfma(kf[ks][1], qf[tt][ks], s[tt][1]);
+            };
+            // First half.  Reads in use order, at most 14 in flight.
+            static_for<0, KS>([&](auto ks) { read_k(ks, kb); });
+            static_for<0, 6>(read_v);
+            const PV8 p0h = p_operand(ph[0]);
+            PV8 p0l = p0h;
+            if constexpr (PSPLIT) p0l = p_operand(pl[0]);
+            softmax(t1, std::integral_constant<int, 0>{}, i);
+            static_for<0, KS>([&](auto ks) {
+                constexpr int k = decltype(ks)::value;
+                lds_wait<2 * (KS - 1 - k) + (k == 0 ? 6 : 8)>(kf[k][0], kf[k][1]);
+                if constexpr (k == 0) { read_v(std::integral_constant<int, 6>{}); read_v(std::integral_constant<int, 7>{}); }
+                qk(t0, ks);
+                softmax(t1, std::integral_constant<int, k + 1>{}, i);
+            });
+            static_for<0, DT>([&](auto dt) {
+                constexpr int d = decltype(dt)::value;
+                lds_wait<DT - 1 - d>(vf[d]);
+                pv(t0, dt, p0h, p0l);
+                if constexpr (d == 2) softmax(t1, std::integral_constant<int, 5>{}, i);
+                if constexpr (d == 5) softmax(t1, std::integral_constant<int, 6>{}, i);
+            });
+            // Second half.
+            const PV8 p1h = p_operand(ph[1]);
+            PV8 p1l = p1h;
+            if constexpr (PSPLIT) p1l = p_operand(pl[1]);
+            static_for<0, KS>([&](auto ks) {
+                constexpr int k = decltype(ks)::value;
+                softmax(t0, ks, i + KG);
+                qk(t1, ks);
+            });
+            static_for<0, DT>([&](auto dt) {
+                constexpr int d = decltype(dt)::value;
+                if constexpr (d % 3 == 0) softmax(t0, std::integral_constant<int, 4 + d / 3>{}, i + KG);
+                pv(t1, dt, p1h, p1l);
+            });
+        }
+    };
+    auto step = [&](int i) __attribute__((always_inline)) {
+        if constexpr (NT == 2) step_two(i);
+        else step_one(i);
     };
 
     // ---- kPrepQuery: the query's hi + lo fragments from its fp32 row ----
@@ -556,7 +669,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             for (int e = 0; e < 8; ++e) {
                 const float x = qx[ks][e >> 2][e & 3];
                 const _Float16 hi = (_Float16)x;
-                qf[ks][e] = hi;
+                qf[0][ks][e] = hi;
                 qlo[ks][e] = (_Float16)(x - (float)hi);
             }
       }
@@ -618,12 +731,14 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     };
 
     // ---- prologue: K0 V0 K1 V1 K2 requested, S^T of page 0 ----
-    s[0] = s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) s[tt][0] = s[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (nl > 0) {
         stage(kh, 0, kring);
         stage(vh, 0, vring);
         if (nl > 1) { stage(kh, 1, kring); stage(vh, 1, vring); }
         if (nl > 2) stage(kh, 2, kring);
+        if (KG == 2 && nl > 3) stage(kh, 3, kring);
     }
     if constexpr (PQ) {
         // Each lane's two RoPE angles depend on the tile's position only, so
@@ -649,13 +764,16 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // meets first).
     auto first_scores = [&]() __attribute__((always_inline)) {
         ring_barrier();
-        static_for<0, KW>([&](auto ks) { read_k(ks, kring_lane); });
-        static_for<0, KS>([&](auto ks) { qk_chunk(ks, kring_lane, s); });
+        const uint32_t kb = kring_lane + kg * PAGE_BYTES;
+        static_for<0, KW>([&](auto ks) { read_k(ks, kb); });
+        static_for<0, KS>([&](auto ks) { qk_chunk(ks, kb, s); });
+        if constexpr (NT == 2)
+            static_for<0, 7>([&](auto part) { softmax(std::integral_constant<int, 0>{}, part, kg); });
     };
     if (nl > 0) {
         // Loader waves: K0 has landed, and the query loads before it.  The
         // others issued no page loads: their query loads.
-        if (w >= kLoaders) wait_vmcnt<0>();
+        if (w >= kLoaders || KG == 2) wait_vmcnt<0>();   // two groups: K1 as well
         else if (nl > 2) wait_vmcnt<4 * H>();
         else if (nl > 1) wait_vmcnt<3 * H>();
         else wait_vmcnt<H>();
@@ -698,12 +816,13 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
                 prepare_v(i);
                 prepare_v(i + 1);
                 ring_barrier();
-                if (i + 3 < nl) stage(kh, i + 3, kring);
-                if (i + 4 < nl) stage(kh, i + 4, kring);
+                // Two groups read K one page further ahead.
+                if (i + KG + 2 < nl) stage(kh, i + KG + 2, kring);
+                if (i + KG + 3 < nl) stage(kh, i + KG + 3, kring);
                 if (i + 2 < nl) stage(vh, i + 2, vring);
                 if (i + 3 < nl) stage(vh, i + 3, vring);
             }
-            if (i < nw) step(i);
+            if (i < nw && (KG == 1 || (i & 1) == kg)) step(i);
         }
     };
     run_pages();
@@ -723,104 +842,141 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             n_keys = wg_keys;
             nl = max(0, (wg_keys + 31) / 32 - p0);
             nw = min(max((wave_keys + 31) / 32 - p0, 0), nl);
-            limit = a.position + row_token;
+            limit[0] = a.position + row_token;
             wave_first_limit = a.position + max(row0, 0) / a.group;
             key_lo = a.position;
             prep_new_keys();
-            s[0] = s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            s[0][0] = s[0][1] = f32x4{0.f, 0.f, 0.f, 0.f};
             if (nl > 0) first_scores();
             run_pages();
         }
     }
 
-    l = row_group_sum(l);
-    const int row = row0 + (lane & 15);
-    if (a.splits > 1) {
-        // ---- partial rows: unnormalised, with their max and sum ----
-        if (row >= 0 && row < row_end) {
-            const size_t part = (size_t)h * a.splits + split;
-            const bool none = m == -INFINITY;   // no key of this split: empty
-            constexpr bool EXACT_V = std::is_same<VT, __bf16>::value;
-            if (!QSPLIT && a.half_parts) {
-                // O / l (a convex combination of V rows: fp16 holds it to
-                // 2^-11 relative when V is fp16).  As in the other 16-bit
-                // partials, lane groups g and g^1 swap halves of each pair
-                // of 16-dim tiles so that every lane stores 8 consecutive
-                // dims (16 B; 64 contiguous bytes per row).  Swap partners
-                // share their row, so both take part or neither does.
-                typedef unsigned U2 __attribute__((ext_vector_type(2)));
-                typedef _Float16 H4 __attribute__((ext_vector_type(4)));
-                const float inv = none ? 0.f : 1.f / l;
-                uint16_t *pa = reinterpret_cast<uint16_t *>(a.part_o) + (part * R + row) * D + 16 * (g & 1) + 4 * (g & 2);
-                uint16_t *pb = pa + (size_t)a.kv_heads * a.splits * R * D;
-                auto store_pair = [&](uint16_t *dst, U2 x, U2 y) __attribute__((always_inline)) {
-                    const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
-                    const auto s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-                    *reinterpret_cast<U4 *>(dst) = U4{s0[0], s1[0], s0[1], s1[1]};
-                };
+    if constexpr (KG == 2) {
+        // ---- merge the two groups: the second leaves its state in LDS ----
+        // Every load has landed (the last meeting's wait); once all waves are
+        // past the barrier no page is read any more.
+        const int wr = w & 3;
+        f32x4 *xacc = reinterpret_cast<f32x4 *>(wr < 2 ? static_cast<void *>(kring) : static_cast<void *>(vring)) +
+                      (wr & 1) * NT * DT * kWave + lane;
+        float *xml = merge_ml + wr * 2 * NT * kWave + lane;
+        wait_vmcnt<0>();
+        lds_barrier();
+        if (kg == 1) {
 #pragma unroll
-                for (int dt = 0; dt < DT; dt += 2) {
-                    const f32x4 x = acc[dt] * inv, y = acc[dt + 1] * inv;
-                    if constexpr (EXACT_V) {
-                        const U4 bx = __builtin_bit_cast(U4, x), by = __builtin_bit_cast(U4, y);
-                        store_pair(pa + dt * 16, U2{(bx[0] >> 16) | (bx[1] & 0xFFFF0000u), (bx[2] >> 16) | (bx[3] & 0xFFFF0000u)},
-                                   U2{(by[0] >> 16) | (by[1] & 0xFFFF0000u), (by[2] >> 16) | (by[3] & 0xFFFF0000u)});
-                        store_pair(pb + dt * 16, U2{(bx[0] & 0xFFFFu) | (bx[1] << 16), (bx[2] & 0xFFFFu) | (bx[3] << 16)},
-                                   U2{(by[0] & 0xFFFFu) | (by[1] << 16), (by[2] & 0xFFFFu) | (by[3] << 16)});
-                    } else {
-                        store_pair(pa + dt * 16,
-                                   __builtin_bit_cast(U2, H4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]}),
-                                   __builtin_bit_cast(U2, H4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]}));
+            for (int tt = 0; tt < NT; ++tt) {
+                xml[2 * tt * kWave] = m[tt];
+                xml[(2 * tt + 1) * kWave] = l[tt];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) xacc[(tt * DT + dt) * kWave] = acc[tt][dt];
+            }
+        }
+        lds_barrier();
+        if (kg == 1) return;
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+            const float m1 = xml[2 * tt * kWave], l1 = xml[(2 * tt + 1) * kWave];
+            const float M = __builtin_fmaxf(m[tt], m1), mu = M == -INFINITY ? 0.f : M;
+            const float f0 = __builtin_amdgcn_exp2f(m[tt] - mu), f1 = __builtin_amdgcn_exp2f(m1 - mu);
+            m[tt] = M;
+            l[tt] = l[tt] * f0 + l1 * f1;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[tt][dt] = acc[tt][dt] * f0 + xacc[(tt * DT + dt) * kWave] * f1;
+        }
+    }
+    static_for<0, NT>([&](auto t_) __attribute__((always_inline)) {
+        constexpr int tt = decltype(t_)::value;
+        l[tt] = row_group_sum(l[tt]);
+        const int row = row0 + 16 * tt + (lane & 15);
+        if (a.splits > 1) {
+            // ---- partial rows: unnormalised, with their max and sum ----
+            if (row >= 0 && row < row_end) {
+                const size_t part = (size_t)h * a.splits + split;
+                const bool none = m[tt] == -INFINITY;   // no key of this split: empty
+                constexpr bool EXACT_V = std::is_same<VT, __bf16>::value;
+                if (!QSPLIT && a.half_parts) {
+                    // O / l (a convex combination of V rows: fp16 holds it to
+                    // 2^-11 relative when V is fp16).  As in the other 16-bit
+                    // partials, lane groups g and g^1 swap halves of each pair
+                    // of 16-dim tiles so that every lane stores 8 consecutive
+                    // dims (16 B; 64 contiguous bytes per row).  Swap partners
+                    // share their row, so both take part or neither does.
+                    typedef unsigned U2 __attribute__((ext_vector_type(2)));
+                    typedef _Float16 H4 __attribute__((ext_vector_type(4)));
+                    const float inv = none ? 0.f : 1.f / l[tt];
+                    uint16_t *pa = reinterpret_cast<uint16_t *>(a.part_o) + (part * R + row) * D + 16 * (g & 1) + 4 * (g & 2);
+                    uint16_t *pb = pa + (size_t)a.kv_heads * a.splits * R * D;
+                    auto store_pair = [&](uint16_t *dst, U2 x, U2 y) __attribute__((always_inline)) {
+                        const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+                        const auto s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+                        *reinterpret_cast<U4 *>(dst) = U4{s0[0], s1[0], s0[1], s1[1]};
+                    };
+#pragma unroll
+                    for (int dt = 0; dt < DT; dt += 2) {
+                        const f32x4 x = acc[tt][dt] * inv, y = acc[tt][dt + 1] * inv;
+                        if constexpr (EXACT_V) {
+                            const U4 bx = __builtin_bit_cast(U4, x), by = __builtin_bit_cast(U4, y);
+                            store_pair(pa + dt * 16, U2{(bx[0] >> 16) | (bx[1] & 0xFFFF0000u), (bx[2] >> 16) | (bx[3] & 0xFFFF0000u)},
+                                       U2{(by[0] >> 16) | (by[1] & 0xFFFF0000u), (by[2] >> 16) | (by[3] & 0xFFFF0000u)});
+                            store_pair(pb + dt * 16, U2{(bx[0] & 0xFFFFu) | (bx[1] << 16), (bx[2] & 0xFFFFu) | (bx[3] << 16)},
+                                       U2{(by[0] & 0xFFFFu) | (by[1] << 16), (by[2] & 0xFFFFu) | (by[3] << 16)});
+                        } else {
+                            store_pair(pa + dt * 16,
+                                       __builtin_bit_cast(U2, H4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]}),
+                                       __builtin_bit_cast(U2, H4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]}));
+                        }
                     }
+                } else {
+                    float *po = a.part_o + (part * R + row) * D + 4 * g;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt)
+                        *reinterpret_cast<f32x4 *>(po + dt * 16) = none ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[tt][dt];
                 }
-            } else {
-                float *po = a.part_o + (part * R + row) * D + 4 * g;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-                    *reinterpret_cast<f32x4 *>(po + dt * 16) = none ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[dt];
+                if (g == 0) {
+                    const float sum = none ? 0.f : l[tt];
+                    a.part_ml[part * 2 * R + row] = m[tt];
+                    a.part_ml[part * 2 * R + R + row] = !QSPLIT && a.half_parts && EXACT_V ? -sum : sum;
+                }
             }
-            if (g == 0) {
-                const float sum = none ? 0.f : l;
-                a.part_ml[part * 2 * R + row] = m;
-                a.part_ml[part * 2 * R + R + row] = !QSPLIT && a.half_parts && EXACT_V ? -sum : sum;
+            return;
+        }
+        // ---- normalise and store rows ----
+        if (row >= 0 && row < row_end) {
+            const int t = row / a.group, gg = row - t * a.group;
+            OUT *dst = static_cast<OUT *>(a.out) + ((size_t)t * a.q_heads + (size_t)h * a.group + gg) * D + 4 * g;
+            const float inv = 1.f / l[tt];
+            // Gated output: times sigmoid(q_gate[t][head][D + d]) (rows of 2D).
+            const float *gate = MODE == kOutGated
+                ? a.gate + ((size_t)t * a.q_heads + (size_t)h * a.group + gg) * 2 * D + D + 4 * g : nullptr;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                typedef OUT OUT4 __attribute__((ext_vector_type(4)));
+                OUT4 o;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = (OUT)(acc[tt][dt][r] * inv);
+                if constexpr (MODE == kOutGated) {
+                    const f32x4 gv = *reinterpret_cast<const f32x4 *>(gate + dt * 16);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[r] *= 1.f / (1.f + expf(-gv[r]));
+                }
+                *reinterpret_cast<OUT4 *>(dst + dt * 16) = o;
             }
         }
-        return;
-    }
-    // ---- normalise and store rows ----
-    if (row >= 0 && row < row_end) {
-        const int t = row / a.group, gg = row - t * a.group;
-        OUT *dst = static_cast<OUT *>(a.out) + ((size_t)t * a.q_heads + (size_t)h * a.group + gg) * D + 4 * g;
-        const float inv = 1.f / l;
-        // Gated output: times sigmoid(q_gate[t][head][D + d]) (rows of 2D).
-        const float *gate = MODE == kOutGated
-            ? a.gate + ((size_t)t * a.q_heads + (size_t)h * a.group + gg) * 2 * D + D + 4 * g : nullptr;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            typedef OUT OUT4 __attribute__((ext_vector_type(4)));
-            OUT4 o;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = (OUT)(acc[dt][r] * inv);
-            if constexpr (MODE == kOutGated) {
-                const f32x4 gv = *reinterpret_cast<const f32x4 *>(gate + dt * 16);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[r] *= 1.f / (1.f + expf(-gv[r]));
-            }
-            *reinterpret_cast<OUT4 *>(dst + dt * 16) = o;
-        }
-    }
+    });
 }
 
 // PREP = kPrepQuery: the fused path's chunk, its query prepared from q_gate
 // (its keys appended by a launch before).
-template <int D, typename KV, typename VT, bool PSPLIT, bool QSPLIT, int MODE, int ROWS, int PREP = 0>
-__global__ __launch_bounds__(ROWS / 16 * kWave, 1)
+template <int D, typename KV, typename VT, bool PSPLIT, bool QSPLIT, int MODE, int ROWS, int PREP = 0, int NT = 1,
+          int KG = 1>
+__global__ __launch_bounds__(ROWS / 16 / NT * KG * kWave, 1)
 void attention_prefill(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) KV kring[4 * 32 * D];
     __shared__ __attribute__((aligned(16))) VT vring[4 * 32 * D];
     __shared__ __attribute__((aligned(16))) float qn_stage[PREP ? ROWS / 16 : 1][PREP ? D : 1];
-    prefill_rows<D, KV, VT, PSPLIT, QSPLIT, MODE, ROWS, -1, PREP>(a, kring, vring, a.v_pages, a.head_stride,
-                                                                  &qn_stage[0][0]);
+    __shared__ float merge_ml[KG == 2 ? ROWS / 16 * 2 * kWave : 1];
+    prefill_rows<D, KV, VT, PSPLIT, QSPLIT, MODE, ROWS, -1, PREP, NT, KG>(a, kring, vring, a.v_pages, a.head_stride,
+                                                                      &qn_stage[0][0], merge_ml);
 }
 
 // The fused prefill chunk that prepares its own query and keys (PREP in
@@ -859,20 +1015,21 @@ void attention_prefill_2pass(PrefillArgs a) {
 // flag multiply by the fp16 copy of V with one fp16 P; a flagged head's take
 // the exact products (bf16 V, P as bf16 hi + lo parts).  Every wave reads
 // the same words, so the choice is uniform.
-template <int D, int MODE, int ROWS>
-__global__ __launch_bounds__(ROWS / 16 * kWave, 1)
+template <int D, int MODE, int ROWS, int NT = 1, int KG = 1>
+__global__ __launch_bounds__(ROWS / 16 / NT * KG * kWave, 1)
 void attention_prefill_bf16(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) __bf16 kring[4 * 32 * D];
     __shared__ __attribute__((aligned(16))) uint16_t vring[4 * 32 * D];
+    __shared__ float merge_ml[KG == 2 ? ROWS / 16 * 2 * kWave : 1];
     const uint32_t *f = a.v_flags + (size_t)(blockIdx.x % a.kv_heads) * a.flag_words;
     uint32_t any = 0;
     for (int i = threadIdx.x & 63; i < a.flag_words; i += 64) any |= f[i];
     if (__any(any != 0))
-        prefill_rows<D, __bf16, __bf16, true, false, MODE, ROWS>(a, kring, reinterpret_cast<__bf16 *>(vring),
-                                                                 a.v_pages, a.head_stride);
+        prefill_rows<D, __bf16, __bf16, true, false, MODE, ROWS, -1, 0, NT, KG>(
+            a, kring, reinterpret_cast<__bf16 *>(vring), a.v_pages, a.head_stride, nullptr, merge_ml);
     else
-        prefill_rows<D, __bf16, _Float16, false, false, MODE, ROWS>(a, kring, reinterpret_cast<_Float16 *>(vring),
-                                                                    a.v_copy, a.v_copy_stride);
+        prefill_rows<D, __bf16, _Float16, false, false, MODE, ROWS, -1, 0, NT, KG>(
+            a, kring, reinterpret_cast<_Float16 *>(vring), a.v_copy, a.v_copy_stride, nullptr, merge_ml);
 }
 
 // Rows per workgroup (kPrefillRows, kernels.hpp): 192 (twelve waves, three
@@ -882,16 +1039,31 @@ void attention_prefill_bf16(PrefillArgs a) {
 // or kPreciseTwoPassRows = 192 on the same eight waves in two passes
 // (attention_prefill_2pass) when that saves rounds of workgroups.
 
+// Raw head_dim 128 calls without key splits take kPairRows = 128 rows per
+// workgroup, two 16-row tiles in each of four waves (step_two), two
+// workgroups per CU (216 VGPRs, 64 KiB of rings each).  Half the LDS reads
+// per row, and vector and matrix work from one wave side by side: 2048 tokens
+// of 32/8/128 at 30,000 1603 -> 1020 us (650 -> 1021 TFLOP/s), 3000 tokens at
+// 0 110.5 -> 84.6 us.  (Other shapes, 3000 tokens at 0: the 16-row tiles in
+// 128-row workgroups, two per CU, 103 us; two tiles in 256 rows, one per CU,
+// 109; three tiles in four waves 100.)  Where every workgroup has a CU of its
+// own, eight waves share its rows, four on the even and four on the odd
+// pages (KG = 2), since four waves cannot fill a CU: 1000 tokens at 3000
+// (256 workgroups) 89.5 -> 74.0 us, 2048 tokens of 8/2/128 33.7 -> 30.8 (192
+// rows in twelve waves: 98.5 and 32.3).  Calls with key splits keep those
+// (few pages per workgroup, where twelve waves' latency counts: 500 bf16
+// tokens of 8/2/128 at 5000 29.6 against 32.5 us with four-wave ones).
+constexpr int kPairRows = 128;
+
 // The raw instances: fp16 pages; bf16 pages, V through the conversion pass
 // below (attention_prefill_bf16).
-template <int D>
+template <int D, int R, int NT, int KG>
 const void *prefill_kernel(Dtype dtype, bool out_f32) {
-    constexpr int R = kPrefillRows;
     if (dtype == Dtype::BF16)
-        return out_f32 ? (const void *)&attention_prefill_bf16<D, kOutF32, R>
-                       : (const void *)&attention_prefill_bf16<D, kOutSame, R>;
-    return out_f32 ? (const void *)&attention_prefill<D, _Float16, _Float16, false, false, kOutF32, R>
-                   : (const void *)&attention_prefill<D, _Float16, _Float16, false, false, kOutSame, R>;
+        return out_f32 ? (const void *)&attention_prefill_bf16<D, kOutF32, R, NT, KG>
+                       : (const void *)&attention_prefill_bf16<D, kOutSame, R, NT, KG>;
+    return out_f32 ? (const void *)&attention_prefill<D, _Float16, _Float16, false, false, kOutF32, R, 0, NT, KG>
+                   : (const void *)&attention_prefill<D, _Float16, _Float16, false, false, kOutSame, R, 0, NT, KG>;
 }
 
 // The fused model path: fp16 pages, fp32 query as hi + lo parts, hi + lo P
@@ -1344,7 +1516,12 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
     a.group = s.group();
     a.rows = s.group() * s.tokens;
     a.position = s.position;
-    a.n_tiles = plan.row_wgs;
+    const bool d256 = s.head_dim == 256;
+    const bool pairs = !precise && !d256 && plan.splits == 1;
+    const int rows = pairs ? kPairRows : plan.rows;
+    const int row_wgs = (a.rows + rows - 1) / rows;
+    const bool groups = pairs && (long long)row_wgs * s.kv_heads <= device_cu_count();
+    a.n_tiles = row_wgs;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.splits = plan.splits;
     if (plan.splits > 1) {
@@ -1353,9 +1530,8 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
         // Raw rows that combine_prefill merges travel as 16-bit planes.
         a.half_parts = !precise && plan.splits <= kCombineWideBatch;
     }
-    const bool d256 = s.head_dim == 256;
-    const int threads = (plan.passes == 2 ? 8 : plan.rows / 16) * kWave;
-    const long long grid = (long long)plan.row_wgs * s.kv_heads * plan.splits;
+    const int threads = (pairs ? (groups ? 8 : 4) : plan.passes == 2 ? 8 : rows / 16) * kWave;
+    const long long grid = (long long)row_wgs * s.kv_heads * plan.splits;
     require(grid * threads < (1LL << 32), "prefill launch exceeds 2^32 work-items");
     void *args[] = {&a};
     auto combine = [&] {
@@ -1389,7 +1565,10 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
         a.v_flags = flags;
         a.flag_words = c.pages;
     }
-    const void *kernel = d256 ? prefill_kernel<256>(dtype, out_f32) : prefill_kernel<128>(dtype, out_f32);
+    const void *kernel = d256     ? prefill_kernel<256, kPrefillRows, 1, 1>(dtype, out_f32)
+                         : !pairs ? prefill_kernel<128, kPrefillRows, 1, 1>(dtype, out_f32)
+                         : groups ? prefill_kernel<128, kPairRows, 2, 2>(dtype, out_f32)
+                                  : prefill_kernel<128, kPairRows, 2, 1>(dtype, out_f32);
     check(hipLaunchKernel(kernel, dim3((unsigned)grid), dim3(threads), args, 0, stream));
     combine();
 }

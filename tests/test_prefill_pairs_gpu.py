@@ -1,0 +1,60 @@
+"""The 128-dim raw prefill (two 16-row tiles per wave; two wave groups over
+alternate pages where every workgroup has a CU of its own) against the oracle
+at the sizes where it can go wrong: a last wave with one row, with one tile
+or with all but one row; one page (the second group has none), two and odd
+page counts; a row max that moves late (outlier keys); negative and zero
+scales; bf16 pages, a flagged KV head among them (the exact products); stale
+slots past the last key hold NaN.  Bounds: max-abs 2e-3, relative L2 1e-3 on
+the fp32 output, as for the other raw calls."""
+import numpy as np
+import pytest
+
+from oracle import attention_ref as ref
+from redshift_amd.workloads import Workload, f32_to_bf16_bits, make_inputs, to_float
+from tests.test_attention_gpu import assert_parity, gpu_attention
+
+pytestmark = pytest.mark.gpu
+
+
+# kv_heads, group, tokens, position.  Up to 256 workgroups of 128 rows (two
+# wave groups on 256 CUs), then more of them (one group, two workgroups a CU).
+GROUPS = [(2, 7, 7, 25), (1, 4, 13, 20), (2, 4, 33, 31), (1, 1, 159, 1), (1, 5, 200, 700),
+          (3, 8, 70, 900)]
+SINGLE = [(8, 4, 1030, 5), (16, 8, 272, 90), (64, 1, 513, 0)]
+
+
+@pytest.mark.parametrize('dtype', ['f16', 'bf16'])
+@pytest.mark.parametrize('kv,group,tokens,position', GROUPS + SINGLE)
+def test_pairs_against_oracle(gpu, kv, group, tokens, position, dtype):
+    w = Workload('pairs', kv * group, kv, 128, tokens, position, 1 / 128 ** .5, dtype, tokens, 1.0, 0.5,
+                 min(8, tokens + position), 8.0)
+    q, k, v, _ = make_inputs(w)
+    want = ref.gqa_attention(to_float(q, dtype), to_float(k, dtype), to_float(v, dtype), position, w.scale)
+    assert_parity(gpu_attention(w, q, k, v, gpu, fill_nan=True, out_dtype=gpu.float32), want)
+
+
+@pytest.mark.parametrize('scale', [-0.07, 0.0, 1e-30])
+@pytest.mark.parametrize('head_dim,kv,group,tokens,position', [(128, 2, 4, 70, 333), (128, 8, 4, 1030, 5),
+                                                               (256, 2, 6, 70, 333)])
+def test_scales_against_oracle(gpu, head_dim, kv, group, tokens, position, scale):
+    w = Workload('scale', kv * group, kv, head_dim, tokens, position, scale, 'f16', 9, 1.0, 0.5)
+    q, k, v, _ = make_inputs(w)
+    want = ref.gqa_attention(to_float(q, 'f16'), to_float(k, 'f16'), to_float(v, 'f16'), position, scale)
+    assert_parity(gpu_attention(w, q, k, v, gpu, fill_nan=True, out_dtype=gpu.float32), want)
+
+
+@pytest.mark.parametrize('kv,group,tokens,position', [(2, 4, 70, 333), (8, 4, 1030, 5)])
+def test_flagged_head_takes_the_exact_products(gpu, kv, group, tokens, position):
+    """KV head 1's values lie far above the fp16 range (2^20 times N(0,1)):
+    its rows are held to the bounds relative to that magnitude."""
+    w = Workload('flagged', kv * group, kv, 128, tokens, position, 1 / 16, 'bf16', 3, 1.0, 1.0)
+    q, k, v, _ = make_inputs(w)
+    v = to_float(v, 'bf16')
+    v[:, 1] *= 2.0 ** 20
+    v = f32_to_bf16_bits(np.ascontiguousarray(v, np.float32))
+    want = ref.gqa_attention(to_float(q, 'bf16'), to_float(k, 'bf16'), to_float(v, 'bf16'), position, w.scale)
+    got = gpu_attention(w, q, k, v, gpu, fill_nan=True, out_dtype=gpu.float32)
+    head = slice(group, 2 * group)
+    assert_parity(got[:, head] / 2.0 ** 20, want[:, head] / 2.0 ** 20)
+    rest = [h for h in range(kv * group) if h not in range(group, 2 * group)]
+    assert_parity(got[:, rest], want[:, rest])
