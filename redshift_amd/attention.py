@@ -2,8 +2,15 @@
 
 torch only supplies device memory and the stream; every computation runs in
 the HIP library.  All calls are stream-ordered on torch's current stream.
+The ordinary forms of `attention` and `attention_fused` are checked, allocated
+and launched by a native extension (csrc/front.cpp); the Python below takes
+the others and raises every error of the checks.
 """
 import ctypes as ct
+import importlib.machinery
+import importlib.util
+import math
+from pathlib import Path
 
 import torch
 
@@ -12,6 +19,26 @@ from .runtime import QV_BF16, QV_F16, QV_F32, check, library
 PAGE_TOKENS = 32
 # Query rows (group * tokens) per KV head that one split/combine pair serves.
 MAX_CHUNK_ROWS = 48
+
+
+FRONT_LIBRARY = Path(__file__).resolve().parent / 'lib' / 'redshift_front.so'
+_FRONT = None
+
+
+def _load_front():
+    """The native calls, bound to the process-wide library (on first use)."""
+    global _FRONT
+    lib = library()
+    if not FRONT_LIBRARY.exists():
+        raise RuntimeError(f'{FRONT_LIBRARY} is missing: build it with `python -m redshift_amd.build`')
+    loader = importlib.machinery.ExtensionFileLoader('redshift_front', str(FRONT_LIBRARY))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader('redshift_front', loader))
+    loader.exec_module(module)
+    module.bind(*[ct.cast(f, ct.c_void_p).value for f in (
+        lib.qv_attention, lib.qv_attention_workspace, lib.qv_attention_fused, lib.qv_attention_fused_workspace,
+        lib.qv_error)], torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+    _FRONT = module
+    return module
 
 
 def dtype_code(dtype):
@@ -47,7 +74,8 @@ def _require(condition, message):
 
 def _same_device(tensors, device):
     for name, t in tensors:
-        _require(t.device == device, f'{name} is on {t.device}, the cache on {device}')
+        if t.device != device:
+            raise ValueError(f'{name} is on {t.device}, the cache on {device}')
 
 
 def _nbytes(t):
@@ -106,6 +134,9 @@ def attention(q, cache, position, scale, out=None, ws=None, out_dtype=None):
     """Raw causal GQA attention: q [tokens][q_heads][head_dim] (cache dtype),
     row t sees keys 0..position+t of `cache` (a PagedKV).  The output has
     q's dtype, or float32 when out_dtype (or out's dtype) says so."""
+    done = (_FRONT or _load_front()).attention(q, cache, position, scale, out, ws, out_dtype)
+    if done is not None:
+        return done
     lib = library()
     _check_query(q, cache)
     q = q.contiguous()
@@ -232,9 +263,10 @@ def check_fused_inputs(q_gate, key, value, q_norm, k_norm, cache):
               'q_norm': (256,), 'k_norm': (256,)}
     named = list(zip(shapes, (q_gate, key, value, q_norm, k_norm)))
     for name, t in named:
-        _require(t.dtype == torch.float32, f'{name} must be float32, not {t.dtype}')
-        _require(t.numel() == torch.Size(shapes[name]).numel(),
-                 f'{name} must hold {shapes[name]} values, not {tuple(t.shape)}')
+        if t.dtype != torch.float32:
+            raise ValueError(f'{name} must be float32, not {t.dtype}')
+        if t.numel() != math.prod(shapes[name]):
+            raise ValueError(f'{name} must hold {shapes[name]} values, not {tuple(t.shape)}')
     _same_device(named, cache.k.device)
     return named
 
@@ -250,6 +282,10 @@ def attention_fused(q_gate, key, value, q_norm, k_norm, cache, position, epsilon
     """Device-side fused attention of the fixed 24/4/256 model (the reference's
     k_attention): prepares q/k, appends k/v at position.., attends and gates.
     All inputs float32 device tensors; `cache` is an fp16 PagedKV(4, 256, ...)."""
+    done = (_FRONT or _load_front()).attention_fused(q_gate, key, value, q_norm, k_norm, cache, position, epsilon,
+                                                     out, ws)
+    if done is not None:
+        return done
     lib = library()
     named = check_fused_inputs(q_gate, key, value, q_norm, k_norm, cache)
     batch = q_gate.shape[0]

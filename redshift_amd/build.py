@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -21,6 +22,10 @@ LIBRARY = PACKAGE / 'lib' / 'libredshift_hip.so'
 # out of the attention library.
 PROBE_SOURCES = ['probe.hip']
 PROBE_LIBRARY = PACKAGE / 'lib' / 'libredshift_probe.so'
+# The torch front end's native calls (a CPython extension against torch's
+# headers; attention.py loads it beside the library, which knows no torch).
+FRONT_SOURCE = PACKAGE / 'csrc' / 'front.cpp'
+FRONT_LIBRARY = PACKAGE / 'lib' / 'redshift_front.so'
 # The commit the library was built from and the library's SHA-256, written
 # beside it by build(), for trees copied without their .git (bench.py's
 # provenance).
@@ -139,9 +144,28 @@ def _link(objects, library):
     os.replace(tmp, library)
 
 
+def build_front():
+    """Compile the torch front end's extension (host code only)."""
+    import torch
+    base = Path(torch.__file__).resolve().parent
+    compiler = shutil.which('g++') or shutil.which('c++')
+    if compiler is None:
+        raise RuntimeError('g++ not found: a host compiler is required to build the torch front end')
+    FRONT_LIBRARY.parent.mkdir(exist_ok=True)
+    tmp = FRONT_LIBRARY.with_suffix('.so.tmp')
+    stderr = _run([compiler, '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall',
+                   f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+                   f'-I{sysconfig.get_paths()["include"]}', f'-I{base / "include"}',
+                   f'-I{base / "include" / "torch" / "csrc" / "api" / "include"}',
+                   str(FRONT_SOURCE), '-o', str(tmp), f'-L{base / "lib"}', '-lc10', '-ltorch_cpu', '-ltorch_python'])
+    os.replace(tmp, FRONT_LIBRARY)
+    return stderr
+
+
 def build(verbose=False, jobs=None):
     """Compile every source and link the shared library (and the probe
-    library beside it); returns the attention library's path."""
+    library and the torch front end beside it); returns the attention
+    library's path."""
     names = SOURCES + PROBE_SOURCES
     results = _compile_all(PACKAGE / '_build', [(name, PACKAGE / 'csrc' / name) for name in names], [], jobs)
     for _, stderr in results:
@@ -150,6 +174,7 @@ def build(verbose=False, jobs=None):
     objects = dict(zip(names, (o for o, _ in results)))
     _link([objects[name] for name in SOURCES], LIBRARY)
     _link([objects[name] for name in PROBE_SOURCES], PROBE_LIBRARY)
+    build_front()
     BUILD_INFO.write_text(json.dumps({'git_head': git_head(),
                                       'library_sha256': hashlib.sha256(LIBRARY.read_bytes()).hexdigest()}) + '\n')
     return LIBRARY

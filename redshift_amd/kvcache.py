@@ -87,15 +87,17 @@ class AttentionKV:
         self._batch = None
         self._recording = False
         self._ws = None
+        self._step_ws = None      # the step's workspace, sized at its first layer
 
     def _ready(self):
         _require(not self.poisoned, 'model state is invalid after a CUDA failure; reset or restore')
 
-    def _workspace(self, batch):
+    def _size_workspace(self, batch):
+        """The step's workspace: every layer of a step needs the same bytes."""
         need = fused_workspace_bytes(batch, self.position)
         if self._ws is None or self._ws.numel() < need:
             self._ws = workspace(need, self.device)
-        return self._ws
+        self._step_ws = self._ws
 
     # -- one evaluated batch ----------------------------------------------
     def begin(self, batch, recording=False):
@@ -118,7 +120,7 @@ class AttentionKV:
         if recording:
             self.verify_position = self.position
         self.poisoned = True
-        self._batch, self._recording = batch, recording
+        self._batch, self._recording, self._step_ws = batch, recording, None
 
     def attend(self, layer, q_gate, key, value, q_norm, k_norm, out=None):
         """k_attention for one full-attention layer (src/runtime.cu:398-407):
@@ -129,9 +131,14 @@ class AttentionKV:
         returns float32 [batch][24][256] (stream-ordered)."""
         _require(self._batch is not None, 'no batch in progress')
         _require(q_gate.shape[0] == self._batch, f'q_gate holds {q_gate.shape[0]} tokens, the batch {self._batch}')
-        check_fused_inputs(q_gate, key, value, q_norm, k_norm, self.caches[layer])
-        return attention_fused(q_gate, key, value, q_norm, k_norm, self.caches[layer], self.position,
-                               self.epsilon, out=out, ws=self._workspace(self._batch))
+        cache = self.caches[layer]
+        if self._step_ws is None:
+            # The step's first layer: its inputs are checked before the
+            # workspace is sized (attention_fused checks every layer's).
+            check_fused_inputs(q_gate, key, value, q_norm, k_norm, cache)
+            self._size_workspace(self._batch)
+        return attention_fused(q_gate, key, value, q_norm, k_norm, cache, self.position, self.epsilon, out=out,
+                               ws=self._step_ws)
 
     def end(self):
         """Finish the batch: the stream is synchronised (the reference's
