@@ -182,7 +182,7 @@ size_t prefill_workspace_bytes(const Shape &s, Dtype dtype, bool precise);
 // rounds over the CUs than 1.5 times those of 192-row ones takes
 // kPreciseTwoPassRows rows per workgroup in two passes of its eight waves
 // (passes = 2): the later 128 rows first, then the earliest 64 rows, which
-// see the fewest keys, on four of the waves.
+// see the fewest keys, two waves on each 16-row tile.
 constexpr int kPrefillRows = 192, kPreciseRows = 128, kPreciseTwoPassRows = 192;
 constexpr int kPrefillMinSplitPages = 8, kPrefillMinSplitKeyPages = 32, kPrefillMaxSplits = 64;
 struct PrefillPlan {

@@ -166,7 +166,7 @@ __device__ __forceinline__ int v_slot_token(int g, int j) {
 // PASS: -1 for a single pass (ROWS / 16 waves, one tile each); 0 and 1 for
 // the two passes of the two-pass instance (eight waves over ROWS = 192 rows:
 // pass 0 gives waves 0-3 the round-0 tiles and waves 4-7 the round-1 tiles,
-// pass 1 gives waves 0-3 the round-2 tiles and waves 4-7 none).
+// pass 1 gives waves w and w + 4 the round-2 tile of slot w, KG = 2).
 // PREP, bit kPrepQuery (the fused path's precise prefill): the query rows
 // are prepared here from q_gate (RMSNorm, gamma, RoPE, hi + lo parts) rather
 // than read as prepared hi + lo parts.  Bit kPrepKeys as well
@@ -201,7 +201,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
                   "the prepared query is the fused model's: fp32 query as hi + lo parts, gated output");
     static_assert(!PK || (PQ && PASS < 0), "the chunk's own keys come with its prepared query, in one pass");
     static_assert(NT == 1 || (PREP == 0 && PASS < 0), "several tiles per wave: the raw instances");
-    static_assert(KG == 1 || (NT == 2 && KG == 2 && kPWaves == 8 && D == 128), "two groups of four waves");
+    static_assert(KG == 1 || (KG == 2 && kPWaves == 8 && ((NT == 2 && D == 128) || PASS == 1)),
+                  "two groups of four waves");
+    static_assert(PASS != 1 || KG == 2, "the second pass has four tiles for eight waves");
     constexpr int KS = D / 32, DT = D / 16;
     constexpr int PAGE = 32 * D;                       // elements of one K (or V) page
     constexpr int PAGE_BYTES = PAGE * 2;
@@ -235,9 +237,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     static_assert(kPWaves % 4 == 0 && kPWaves / 4 <= 3, "one to three rounds of four waves");
     const int T = (R + TR - 1) / TR, K = 4 * a.n_tiles, slot = 4 * j + (w & 3);
     const int kg = KG == 1 ? 0 : w >> 2;                      // this wave's pages: kg, kg + KG, ...
-    const int round = PASS == 1 ? (w < 4 ? 2 : 3) : KG == 1 ? w >> 2 : 0;   // round 3: no tile
+    const int round = PASS == 1 ? 2 : KG == 1 ? w >> 2 : 0;
     const int tile = round == 0 ? T - 1 - slot : round == 1 ? T - 2 * K + slot
-                   : round == 2 ? T - 3 * K + slot : -1;
+                                : T - 3 * K + slot;
     const int row0 = TR * tile;
     const int row_end = R;                                              // valid rows: [0, row_end)
 
@@ -486,7 +488,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // computed from a stale buffer and dropped.)
     auto step_one = [&](int i) __attribute__((always_inline)) {
         if constexpr (NT == 1) {
-            const uint32_t kb = kring_lane + ((i + 1) & 3) * PAGE_BYTES;
+            const uint32_t kb = kring_lane + ((i + KG) & 3) * PAGE_BYTES;
             const uint32_t vb = vring_lane + (i & 3) * PAGE_BYTES;
             f32x4 sn[1][2] = {{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}};
             // The S^T and softmax phase runs at raised wave priority, the P.V
@@ -755,6 +757,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
         // wait for them alone and prepare the query while the pages are in
         // flight.
         if (w >= kLoaders || nl == 0) wait_vmcnt<0>();
+        else if (KG == 2 && nl > 3) wait_vmcnt<6 * H>();
         else if (nl > 2) wait_vmcnt<5 * H>();
         else if (nl > 1) wait_vmcnt<4 * H>();
         else wait_vmcnt<2 * H>();
@@ -857,8 +860,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
         // Every load has landed (the last meeting's wait); once all waves are
         // past the barrier no page is read any more.
         const int wr = w & 3;
-        f32x4 *xacc = reinterpret_cast<f32x4 *>(wr < 2 ? static_cast<void *>(kring) : static_cast<void *>(vring)) +
-                      (wr & 1) * NT * DT * kWave + lane;
+        constexpr int PER = PAGE_BYTES * 4 / (NT * DT * kWave * 16);   // waves per ring: 2, or 4 (one tile)
+        f32x4 *xacc = reinterpret_cast<f32x4 *>(wr < PER ? static_cast<void *>(kring) : static_cast<void *>(vring)) +
+                      wr % PER * NT * DT * kWave + lane;
         float *xml = merge_ml + wr * 2 * NT * kWave + lane;
         wait_vmcnt<0>();
         lds_barrier();
@@ -993,8 +997,12 @@ void attention_prefill_prep(PrefillArgs a) {
 }
 
 // The precise rows in two passes of eight waves (192 rows per workgroup):
-// one round of workgroups where 128-row ones would take two.  Between the
-// passes every wave's output stores complete (the second pass's waits count
+// one round of workgroups where 128-row ones would take two.  The second
+// pass has four tiles: two waves share each, one on the even and one on the
+// odd pages, so that every SIMD keeps two waves (the fused 2048-token chunk at
+// 6144 612.6 -> 593.7 us against four waves with a tile each; two waves on the
+// key halves of every page repeat its softmax steps and were slower than
+// either).  Between the passes every wave's output stores complete (the second pass's waits count
 // its page loads only) and every wave has finished reading the rings.
 template <int D, typename KV, typename VT, bool PSPLIT, bool QSPLIT, int MODE, int PREP = 0>
 __global__ __launch_bounds__(8 * kWave, 1)
@@ -1003,12 +1011,13 @@ void attention_prefill_2pass(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) KV kring[4 * 32 * D];
     __shared__ __attribute__((aligned(16))) VT vring[4 * 32 * D];
     __shared__ __attribute__((aligned(16))) float qn_stage[PREP ? 8 : 1][PREP ? D : 1];
+    __shared__ float merge_ml[4 * 2 * kWave];
     prefill_rows<D, KV, VT, PSPLIT, QSPLIT, MODE, ROWS, 0, PREP>(a, kring, vring, a.v_pages, a.head_stride,
                                                                  &qn_stage[0][0]);
     wait_vmcnt<0>();
     ring_barrier();
-    prefill_rows<D, KV, VT, PSPLIT, QSPLIT, MODE, ROWS, 1, PREP>(a, kring, vring, a.v_pages, a.head_stride,
-                                                                 &qn_stage[0][0]);
+    prefill_rows<D, KV, VT, PSPLIT, QSPLIT, MODE, ROWS, 1, PREP, 1, 2>(a, kring, vring, a.v_pages, a.head_stride,
+                                                                       &qn_stage[0][0], merge_ml);
 }
 
 // bf16 pages: the workgroups of a KV head that the conversion pass did not

@@ -1,17 +1,19 @@
-"""The 128-dim raw prefill (two 16-row tiles per wave; two wave groups over
-alternate pages where every workgroup has a CU of its own) against the oracle
-at the sizes where it can go wrong: a last wave with one row, with one tile
-or with all but one row; one page (the second group has none), two and odd
-page counts; a row max that moves late (outlier keys); negative and zero
-scales; bf16 pages, a flagged KV head among them (the exact products); stale
-slots past the last key hold NaN.  Bounds: max-abs 2e-3, relative L2 1e-3 on
-the fp32 output, as for the other raw calls."""
+"""The prefill instances whose waves share rows: the 128-dim raw prefill (two
+16-row tiles per wave; two wave groups over alternate pages where every
+workgroup has a CU of its own) and the second pass of the two-pass precise
+prefill, against the oracle at the sizes where they can go wrong: a last wave
+with one row, with one tile or with all but one row; one page (the second
+group has none), two and odd page counts; a row max that moves late (outlier
+keys); negative and zero scales; bf16 pages, a flagged KV head among them (the
+exact products); stale slots past the last key hold NaN.  Bounds: max-abs
+2e-3, relative L2 1e-3 on the fp32 output, as for the other raw calls."""
 import numpy as np
 import pytest
 
 from oracle import attention_ref as ref
 from redshift_amd.workloads import Workload, f32_to_bf16_bits, make_inputs, to_float
 from tests.test_attention_gpu import assert_parity, gpu_attention
+from tests.test_configs_gpu import PRECISE_REL_L2, precise_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +60,20 @@ def test_flagged_head_takes_the_exact_products(gpu, kv, group, tokens, position)
     assert_parity(got[:, head] / 2.0 ** 20, want[:, head] / 2.0 ** 20)
     rest = [h for h in range(kv * group) if h not in range(group, 2 * group)]
     assert_parity(got[:, rest], want[:, rest])
+
+
+@pytest.mark.parametrize('head_dim', [128, 256])
+@pytest.mark.parametrize('tokens,position', [(129, 0), (150, 0), (177, 40), (192, 1), (161, 500)])
+def test_precise_two_passes_against_oracle(gpu, head_dim, tokens, position):
+    """200 KV heads of 129..192 rows: 192 rows per workgroup in two passes
+    (one round of workgroups instead of two), whose second takes the earliest
+    rows on two wave groups over alternate pages: padded tiles, a second
+    pass over one page, two and more.  Bounds of the precise entry."""
+    w = Workload('two_pass', 200, 200, head_dim, tokens, position, 1 / head_dim ** .5, 'f32', tokens, 1.0, 0.5,
+                 min(8, position + tokens), 8.0)
+    q, k, v, _ = make_inputs(w)
+    k16, v16 = k.astype(np.float16), v.astype(np.float16)
+    got = precise_attention(w, q, k16, v16, gpu)
+    want = ref.gqa_attention(q, k16, v16, position, w.scale)
+    assert_parity(got, want)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) <= PRECISE_REL_L2
