@@ -1048,20 +1048,29 @@ void attention_prefill_bf16(PrefillArgs a) {
 // or kPreciseTwoPassRows = 192 on the same eight waves in two passes
 // (attention_prefill_2pass) when that saves rounds of workgroups.
 
-// Raw head_dim 128 calls without key splits take kPairRows = 128 rows per
-// workgroup, two 16-row tiles in each of four waves (step_two), two
-// workgroups per CU (216 VGPRs, 64 KiB of rings each).  Half the LDS reads
-// per row, and vector and matrix work from one wave side by side: 2048 tokens
-// of 32/8/128 at 30,000 1603 -> 1020 us (650 -> 1021 TFLOP/s), 3000 tokens at
-// 0 110.5 -> 84.6 us.  (Other shapes, 3000 tokens at 0: the 16-row tiles in
-// 128-row workgroups, two per CU, 103 us; two tiles in 256 rows, one per CU,
-// 109; three tiles in four waves 100.)  Where every workgroup has a CU of its
-// own, eight waves share its rows, four on the even and four on the odd
-// pages (KG = 2), since four waves cannot fill a CU: 1000 tokens at 3000
-// (256 workgroups) 89.5 -> 74.0 us, 2048 tokens of 8/2/128 33.7 -> 30.8 (192
-// rows in twelve waves: 98.5 and 32.3).  Calls with key splits keep those
-// (few pages per workgroup, where twelve waves' latency counts: 500 bf16
-// tokens of 8/2/128 at 5000 29.6 against 32.5 us with four-wave ones).
+// Raw head_dim 128 calls without key splits have two more instances, of
+// kPairRows = 128 rows per workgroup, two 16-row tiles in each of four waves
+// (step_two).  All three reach about the same rate on a full device (3072
+// fp16 tokens of 32/8/128 at 20,000: 1060 us, 1.02 PFLOP/s, in two rounds of
+// 192-row workgroups or three of 128-row pairs); what differs is how well
+// their workgroups fill it.
+//   192 rows, twelve waves: the serpentine deal gives every workgroup the same
+//     work, but a round of workgroups that is not full is lost whole.  Taken
+//     for one round at most (1100 tokens at 3000: 91.2 against 104.9 us with
+//     pairs; 1500 at 0: 32.1 against 39.3).
+//   Pairs, four waves (216 VGPRs, 64 KiB of rings: two workgroups per CU):
+//     several rounds, the longest workgroups first and the CUs refilled as
+//     they end (2048 at 30,000: 999 us, 192-row workgroups 1581; 3000 at
+//     0: 83.1 against 107.8; 1600 at 3000: 120.6 against 176.3).
+//   Pairs in two groups of four waves, on the even and the odd pages (KG = 2):
+//     where every 128-row workgroup has a CU of its own, four waves alone
+//     would leave it half empty (1000 at 3000: 72.3 us, 89.5 with four waves,
+//     83.5 with the 192-row workgroups).  A prefix shorter than a quarter of
+//     the chunk keeps the 192-row deal, since the last rows' workgroup, with
+//     its many keys, then sets the time (1000 at 200: 28.1 and 28.0 us; 1000
+//     at 0: 25.1 against 24.1; 4000 of 8/2/128 at 0: 70.1 against 66.2).
+// Calls with key splits run few pages per workgroup and keep twelve waves (500
+// bf16 tokens of 8/2/128 at 5000: 29.6 against 32.5 us with pairs).
 constexpr int kPairRows = 128;
 
 // The raw instances: fp16 pages; bf16 pages, V through the conversion pass
@@ -1526,10 +1535,14 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
     a.rows = s.group() * s.tokens;
     a.position = s.position;
     const bool d256 = s.head_dim == 256;
-    const bool pairs = !precise && !d256 && plan.splits == 1;
+    // See kPairRows.
+    const int cus = device_cu_count();
+    const bool may_pair = !precise && !d256 && plan.splits == 1;
+    const long long pair_wgs = (a.rows + (long long)kPairRows - 1) / kPairRows * s.kv_heads;
+    const bool groups = may_pair && pair_wgs <= cus && 4LL * s.position >= s.tokens;
+    const bool pairs = groups || (may_pair && (long long)plan.row_wgs * s.kv_heads > cus);
     const int rows = pairs ? kPairRows : plan.rows;
     const int row_wgs = (a.rows + rows - 1) / rows;
-    const bool groups = pairs && (long long)row_wgs * s.kv_heads <= device_cu_count();
     a.n_tiles = row_wgs;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.splits = plan.splits;

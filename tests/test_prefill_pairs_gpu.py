@@ -18,15 +18,17 @@ from tests.test_configs_gpu import PRECISE_REL_L2, precise_attention
 pytestmark = pytest.mark.gpu
 
 
-# kv_heads, group, tokens, position.  Up to 256 workgroups of 128 rows (two
-# wave groups on 256 CUs), then more of them (one group, two workgroups a CU).
-GROUPS = [(2, 7, 7, 25), (1, 4, 13, 20), (2, 4, 33, 31), (1, 1, 159, 1), (1, 5, 200, 700),
+# kv_heads, group, tokens, position.  Up to 256 workgroups of 128 rows after a
+# prefix (two wave groups on 256 CUs); more than 256 workgroups of 192 rows (one
+# group, two workgroups a CU); one round of 192-row workgroups.
+GROUPS = [(1, 8, 7, 2), (2, 7, 7, 25), (1, 4, 13, 20), (2, 4, 33, 31), (1, 1, 159, 40), (1, 5, 200, 700),
           (3, 8, 70, 900)]
-SINGLE = [(8, 4, 1030, 5), (16, 8, 272, 90), (64, 1, 513, 0)]
+SINGLE = [(8, 4, 1540, 5), (130, 1, 193, 0), (130, 1, 257, 40), (65, 2, 400, 600)]
+ROUND = [(1, 1, 159, 1), (8, 4, 200, 0)]
 
 
 @pytest.mark.parametrize('dtype', ['f16', 'bf16'])
-@pytest.mark.parametrize('kv,group,tokens,position', GROUPS + SINGLE)
+@pytest.mark.parametrize('kv,group,tokens,position', GROUPS + SINGLE + ROUND)
 def test_pairs_against_oracle(gpu, kv, group, tokens, position, dtype):
     w = Workload('pairs', kv * group, kv, 128, tokens, position, 1 / 128 ** .5, dtype, tokens, 1.0, 0.5,
                  min(8, tokens + position), 8.0)
@@ -36,7 +38,7 @@ def test_pairs_against_oracle(gpu, kv, group, tokens, position, dtype):
 
 
 @pytest.mark.parametrize('scale', [-0.07, 0.0, 1e-30])
-@pytest.mark.parametrize('head_dim,kv,group,tokens,position', [(128, 2, 4, 70, 333), (128, 8, 4, 1030, 5),
+@pytest.mark.parametrize('head_dim,kv,group,tokens,position', [(128, 2, 4, 70, 333), (128, 130, 1, 193, 0),
                                                                (256, 2, 6, 70, 333)])
 def test_scales_against_oracle(gpu, head_dim, kv, group, tokens, position, scale):
     w = Workload('scale', kv * group, kv, head_dim, tokens, position, scale, 'f16', 9, 1.0, 0.5)
@@ -45,7 +47,7 @@ def test_scales_against_oracle(gpu, head_dim, kv, group, tokens, position, scale
     assert_parity(gpu_attention(w, q, k, v, gpu, fill_nan=True, out_dtype=gpu.float32), want)
 
 
-@pytest.mark.parametrize('kv,group,tokens,position', [(2, 4, 70, 333), (8, 4, 1030, 5)])
+@pytest.mark.parametrize('kv,group,tokens,position', [(2, 4, 70, 333), (130, 1, 193, 0)])
 def test_flagged_head_takes_the_exact_products(gpu, kv, group, tokens, position):
     """KV head 1's values lie far above the fp16 range (2^20 times N(0,1)):
     its rows are held to the bounds relative to that magnitude."""
