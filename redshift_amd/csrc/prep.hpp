@@ -70,8 +70,9 @@ __device__ __forceinline__ float lane_xor32(float x) {
 // multiply-adds is off here, since the compiler would otherwise pick which
 // product to fuse per call site, and a K row appended to the cache must have
 // the same bits whichever kernel instance prepared it.
+// (gamma of each row, or one for all of them: norm_rope_rows below.)
 template <int R>
-__device__ __forceinline__ void norm_rope_rows(float (&x)[R][4], const float (&gamma)[4], const float (&c)[R],
+__device__ __forceinline__ void norm_rope_each(float (&x)[R][4], const float (&gamma)[R][4], const float (&c)[R],
                                                const float (&s)[R], float epsilon, int lane) {
 #pragma clang fp contract(off)
     constexpr float kInvD = 1.f / (4 * kWave);
@@ -88,7 +89,7 @@ __device__ __forceinline__ void norm_rope_rows(float (&x)[R][4], const float (&g
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) x[r][w] = ((x[r][w] * inv[r]) * gamma[w]);
+        for (int w = 0; w < 4; ++w) x[r][w] = ((x[r][w] * inv[r]) * gamma[r][w]);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const float other = lane_xor32(x[r][0]);
@@ -96,6 +97,17 @@ __device__ __forceinline__ void norm_rope_rows(float (&x)[R][4], const float (&g
         x[r][0] = lane < 32 ? ((x[r][0] * c[r]) - (other * s[r]))    // a c - b s
                             : ((other * sp) + (x[r][0] * cp));    // a s + b c
     }
+}
+
+template <int R>
+__device__ __forceinline__ void norm_rope_rows(float (&x)[R][4], const float (&gamma)[4], const float (&c)[R],
+                                               const float (&s)[R], float epsilon, int lane) {
+    float g[R][4];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) g[r][w] = gamma[w];
+    norm_rope_each<R>(x, g, c, s, epsilon, lane);
 }
 
 // The fused split kernels' new keys: the inputs of new token j's key for

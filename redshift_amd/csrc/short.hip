@@ -21,13 +21,22 @@
 //     independent accumulations, O^T += V^T.P^T, P as fp16 hi + lo, online
 //     softmax in base 2); position + tokens <= 256 leaves at most one wave
 //     with a second page;
-//   * every wave rescales its partial O to the workgroup's row maxima, waves
-//     4..7 hand theirs to waves 0..3 through LDS, and each thread sums the
-//     four remaining partials of one output element and writes it gated:
-//     out = O / L * sigmoid(gate).
+//   * every wave with a page leaves its row maxima, sums and partial O in a
+//     slot of LDS of its own, and after one barrier each thread merges one
+//     output element and writes it gated: out = O / L * sigmoid(gate).
+// The tokens' workgroups of a KV head read the same pages at the same time,
+// so the grid puts a head's workgroups on the same two XCDs (id i runs on
+// XCD i % 8; heads vary fastest) and the page loads keep the default policy:
+// one workgroup's miss then serves the others from that XCD's L2.  Per layer
+// in a graph, 8 tokens after 16, 100 and 248 keys: 8.97, 11.09 and 14.38 us
+// with tokens fastest and non-temporal loads; 7.17, 9.64 and 13.06 with the
+// query row and the new key prepared side by side and the one-barrier merge
+// (before: one after the other, and three barriers); 6.34, 8.18 and 10.16 with
+// heads fastest as well; 6.03, 7.38 and 8.83 with default-policy loads.
 // Cached-page slots from `position` on are masked and their values zeroed:
 // other workgroups append the new tokens there while this one reads.
 #include "kernels.hpp"
+#include "lds.hpp"
 #include "prep.hpp"
 
 #include <cmath>
@@ -57,7 +66,6 @@ void attention_fused_short(ShortArgs a) {
     constexpr int D = kModelHeadDim, H = kModelQHeads, HKV = kModelKvHeads, G = H / HKV;
     constexpr int KS = D / 32, DT = D / 16, PAGE = 32 * D;
     constexpr int NE = G * D / 4;               // output elements (f32x4) of the workgroup
-    constexpr int kHalf = kShortWaves / 2;
     static_assert(D == 4 * kWave, "256-dim rows, four values per lane");
     static_assert(kShortWaves == kShortMaxTokens && G <= kShortWaves, "one query row and one new key per wave");
     static_assert(NE <= kShortWaves * kWave, "one output element per thread");
@@ -66,29 +74,29 @@ void attention_fused_short(ShortArgs a) {
     // part 1 = fp16(q - part 0); rows past the group are zero.
     __shared__ f16x8 qf[2][KS][kWave];
     __shared__ __attribute__((aligned(16))) _Float16 knew[PAGE], vnew[PAGE];   // the new keys' page
-    __shared__ f32x4 so[kHalf][DT * kWave];     // partial O of waves 4..7, then of the pairs
+    __shared__ f32x4 so[kShortWaves][DT * 4 * G];   // each wave's partial O
     __shared__ float sml[kShortWaves][2][16];
 
     const FusedToken &tok = a.tok;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int t = blockIdx.x, h = blockIdx.y;
+    const int t = blockIdx.y, h = blockIdx.x;
     const int position = tok.position;          // cached keys 0 .. position-1
     const int n_cached = (position + 31) / 32;  // cached pages; page n_cached is the new keys'
     const bool has_q = w < G, has_key = w <= t;   // wave-uniform
 
     // ---- every load first (lane l holds dims 64i + l of a row); rows a wave
     // does not use are read at a clamped index so every address is valid ----
-    float xq[1][4], xk[1][4], xv[4], gq[4], gk[4];
+    float x2[2][4], g2[2][4], xv[4];   // the query row and the new key, and their norms' weights
     {
         const float *qs = tok.q_gate + ((size_t)t * H + h * G + min(w, G - 1)) * 2 * D;
         const size_t kr = ((size_t)min(w, t) * HKV + h) * D;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            xq[0][i] = qs[64 * i + lane];
-            xk[0][i] = tok.key[kr + 64 * i + lane];
+            x2[0][i] = qs[64 * i + lane];
+            x2[1][i] = tok.key[kr + 64 * i + lane];
             xv[i] = tok.value[kr + 64 * i + lane];
-            gq[i] = tok.q_norm[64 * i + lane];
-            gk[i] = tok.k_norm[64 * i + lane];
+            g2[0][i] = tok.q_norm[64 * i + lane];
+            g2[1][i] = tok.k_norm[64 * i + lane];
         }
     }
     // The gate of this thread's output element e: row e / 64, dims
@@ -105,10 +113,10 @@ void attention_fused_short(ShortArgs a) {
         for (int tile = 0; tile < 2; ++tile)
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
-                kb[tile][ks] = __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(kp + tile * 16 * D + ks * 512));
+                kb[tile][ks] = *reinterpret_cast<const f16x8 *>(kp + tile * 16 * D + ks * 512);
         const _Float16 *vp = vh + (size_t)w * PAGE;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vb[dt] = __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(vp + dt * 512));
+        for (int dt = 0; dt < DT; ++dt) vb[dt] = *reinterpret_cast<const f16x8 *>(vp + dt * 512);
     }
     // Zero the fragments of rows G..15 (lanes 16g + r, r >= G), which no
     // wave prepares: KS*4*(16-G) entries per part.
@@ -118,12 +126,16 @@ void attention_fused_short(ShortArgs a) {
         qf[part][ks][16 * g + r] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
 
-    // ---- prepare this wave's query row and new key ----
+    // ---- prepare this wave's query row and new key (side by side: a wave
+    // without the one or the other prepares a clamped row and drops it) ----
     const double freq = rope_freq(lane);
+    float c2[2] = {1.f, 1.f}, s2[2] = {0.f, 0.f};
+    if (lane < 32) {
+        rope_cos_sin(position + t, freq, c2[0], s2[0]);
+        rope_cos_sin(position + w, freq, c2[1], s2[1]);
+    }
+    norm_rope_each<2>(x2, g2, c2, s2, tok.epsilon, lane);
     if (has_q) {
-        float c[1] = {1.f}, s[1] = {0.f};
-        if (lane < 32) rope_cos_sin(position + t, freq, c[0], s[0]);
-        norm_rope_rows<1>(xq, gq, c, s, tok.epsilon, lane);
         // Dim d = 64i + l of row w: k-step d / 32, lane 16 ((d % 32) / 8) + w,
         // element d % 8.
         _Float16 *qh = reinterpret_cast<_Float16 *>(&qf[0][0][0]);
@@ -131,20 +143,17 @@ void attention_fused_short(ShortArgs a) {
         for (int i = 0; i < 4; ++i) {
             const int d = 64 * i + lane;
             const int at = ((d >> 5) * kWave + 16 * ((d >> 3) & 3) + w) * 8 + (d & 7);
-            const _Float16 hi = (_Float16)xq[0][i];
+            const _Float16 hi = (_Float16)x2[0][i];
             qh[at] = hi;
-            qh[KS * kWave * 8 + at] = (_Float16)(xq[0][i] - (float)hi);
+            qh[KS * kWave * 8 + at] = (_Float16)(x2[0][i] - (float)hi);
         }
     }
     if (has_key) {
-        float c[1] = {1.f}, s[1] = {0.f};
-        if (lane < 32) rope_cos_sin(position + w, freq, c[0], s[0]);
-        norm_rope_rows<1>(xk, gk, c, s, tok.epsilon, lane);
         _Float16 *kp = static_cast<_Float16 *>(tok.k_pages) + (size_t)h * tok.head_stride;
         _Float16 *vp = static_cast<_Float16 *>(tok.v_pages) + (size_t)h * tok.head_stride;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const _Float16 kq = cache_half(xk[0][i]), vq = cache_half(xv[i]);
+            const _Float16 kq = cache_half(x2[1][i]), vq = cache_half(xv[i]);
             knew[k_page_offset(w, 64 * i + lane, D)] = kq;
             vnew[v_page_offset(w, 64 * i + lane, D)] = vq;
             if (w == t) {
@@ -188,8 +197,7 @@ void attention_fused_short(ShortArgs a) {
         float bm = x[0];
 #pragma unroll
         for (int j = 1; j < 8; ++j) bm = fmaxf(bm, x[j]);
-        bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
+        bm = row_group_max(bm);
         const float mn = fmaxf(m, bm);   // finite: every page has a valid key
         const float alpha = __builtin_amdgcn_exp2f(m - mn);
         m = mn;
@@ -237,49 +245,45 @@ void attention_fused_short(ShortArgs a) {
     }
 
     // ---- merge the waves and write the gated rows ----
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
-    if (lane < 16) {
-        sml[w][0][lane] = m;
-        sml[w][1][lane] = l;
-    }
-    lds_barrier();
-    // Row r = l % 16 of lane l: the workgroup's maximum, finite for every
-    // row (key t is always seen; rows past the group have zero scores).  A
-    // wave without pages has m = -inf and acc = 0 and adds nothing.
-    {
+    // One barrier: every wave with a page leaves its (m, l) and the group's
+    // rows of its unscaled accumulators in a slot of its own ([fragment][lane
+    // group][row], so the stores are contiguous and the reads below free of
+    // bank conflicts); then each thread merges one output element.
+    const int used = min(n_cached + 1, kShortWaves);   // waves with pages: 0 .. used-1
+    if (w < used) {
+        l = row_group_sum(l);
         const int r = lane & 15;
-        float M = sml[0][0][r];
+        if (lane < 16) {
+            sml[w][0][lane] = m;
+            sml[w][1][lane] = l;
+        }
+        if (r < G) {
 #pragma unroll
-        for (int ww = 1; ww < kShortWaves; ++ww) M = fmaxf(M, sml[ww][0][r]);
-        const float f = __builtin_amdgcn_exp2f(m - M);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] *= f;
-    }
-    if (w >= kHalf) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) so[w - kHalf][dt * kWave + lane] = acc[dt];
+            for (int dt = 0; dt < DT; ++dt) so[w][(dt * 4 + (lane >> 4)) * G + r] = acc[dt];
+        }
     }
     lds_barrier();
-    if (w < kHalf) {
-        // Each slot is read and rewritten by the same lanes of one wave.
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) so[w][dt * kWave + lane] += acc[dt];
-    }
-    lds_barrier();
-    // Element e: row e / 64, dims 4 (e % 64) .. +3, which is the f32x4 of
-    // lane r + 16 (d4 % 4) in fragment d4 / 4 of every slot.
+    // Element e: row e / 64, dims 4 (e % 64) .. +3: fragment (e % 64) / 4,
+    // lane group e % 4.  Every wave with a page has a finite max for every
+    // row (each page has a valid key).
     if ((int)threadIdx.x < NE) {
         const int r = e / 64, d4 = e % 64;
-        float M = sml[0][0][r];
+        float mw[kShortWaves], M = sml[0][0][r];
 #pragma unroll
-        for (int ww = 1; ww < kShortWaves; ++ww) M = fmaxf(M, sml[ww][0][r]);
+        for (int ww = 0; ww < kShortWaves; ++ww) {
+            mw[ww] = sml[min(ww, used - 1)][0][r];
+            M = fmaxf(M, mw[ww]);
+        }
         float L = 0.f;
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ww = 0; ww < kShortWaves; ++ww) L += sml[ww][1][r] * __builtin_amdgcn_exp2f(sml[ww][0][r] - M);
-        f32x4 o = so[0][(d4 >> 2) * kWave + r + 16 * (d4 & 3)];
-#pragma unroll
-        for (int s = 1; s < kHalf; ++s) o += so[s][(d4 >> 2) * kWave + r + 16 * (d4 & 3)];
+        for (int ww = 0; ww < kShortWaves; ++ww) {
+            if (ww < used) {
+                const float f = __builtin_amdgcn_exp2f(mw[ww] - M);
+                L += sml[ww][1][r] * f;
+                o += so[ww][d4 * G + r] * f;
+            }
+        }
         const float inv = 1.f / L;
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] *= inv * (1.f / (1.f + expf(-gate[j])));
@@ -297,7 +301,7 @@ void launch_fused_short(const FusedToken &tok, float *out, hipStream_t stream) {
     a.out = out;
     a.scale_log2 = (1.0f / 16.0f) * 1.4426950408889634f;
     void *args[] = {&a};
-    check(hipLaunchKernel((const void *)&attention_fused_short, dim3(tok.tokens, kModelKvHeads),
+    check(hipLaunchKernel((const void *)&attention_fused_short, dim3(kModelKvHeads, tok.tokens),
                           dim3(kShortWaves * kWave), args, 0, stream));
 }
 
