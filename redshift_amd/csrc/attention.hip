@@ -168,7 +168,9 @@ void attention_stream(SplitArgs a) {
     __shared__ float sml[kWaves][2][16];
 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int split = blockIdx.x % a.splits, h = blockIdx.x / a.splits;
+    // Heads fastest, as in attention_ring (raw decode at 4,095 keys 9.58 -> 9.50
+    // us per call in a graph, the fused decode at 139,263 87.70 -> 87.56).
+    const int h = blockIdx.x % a.kv_heads, split = blockIdx.x / a.kv_heads;
     QS qs;
     // PREP: rows 3w + r of token w/2 (lane l holding dims 64i + l), and the
     // new key of token w in the first split.
@@ -654,7 +656,7 @@ void launch_split(const Shape &s, const SplitPlan &plan, Dtype dtype, bool preci
     }
     const void *kernel = split_kernel(plan, s.head_dim, dtype, precise, out_mode);
     void *args[] = {&a};
-    // One-dimensional grid: workgroup id = KV head * splits + split.
+    // One-dimensional grid: workgroup id = split * KV heads + KV head.
     check(hipLaunchKernel(kernel, dim3(plan.splits * s.kv_heads), dim3(block_threads(plan)),
                           args, 0, stream));
 }
