@@ -168,9 +168,10 @@ void attention_stream(SplitArgs a) {
     __shared__ float sml[kWaves][2][16];
 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    // Heads fastest, as in attention_ring (raw decode at 4,095 keys 9.58 -> 9.50
-    // us per call in a graph, the fused decode at 139,263 87.70 -> 87.56).
-    const int h = blockIdx.x % a.kv_heads, split = blockIdx.x / a.kv_heads;
+    // Splits fastest (heads fastest, as in attention_ring, gave 16.97 against
+    // 16.82 us per call at 16,391 keys, 16 cold caches in a graph: a decode has
+    // few query rows to share, and a head's stream spreads over every XCD).
+    const int split = blockIdx.x % a.splits, h = blockIdx.x / a.splits;
     QS qs;
     // PREP: rows 3w + r of token w/2 (lane l holding dims 64i + l), and the
     // new key of token w in the first split.
@@ -656,7 +657,7 @@ void launch_split(const Shape &s, const SplitPlan &plan, Dtype dtype, bool preci
     }
     const void *kernel = split_kernel(plan, s.head_dim, dtype, precise, out_mode);
     void *args[] = {&a};
-    // One-dimensional grid: workgroup id = split * KV heads + KV head.
+    // One-dimensional grid over (KV head, split); each kernel orders it itself.
     check(hipLaunchKernel(kernel, dim3(plan.splits * s.kv_heads), dim3(block_threads(plan)),
                           args, 0, stream));
 }
