@@ -314,6 +314,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     const int wave_last = min(row0 + TR - 1, row_end - 1);
     const int wave_keys = wave_last < max(row0, 0) ? 0 : a.position + wave_last / a.group + 1;
     int nw = min(max((PK && wave_keys ? n : (wave_keys + 31) / 32) - p0, 0), nl);
+    // Two tiles: those of its first tile alone, which may end a page earlier.
+    [[maybe_unused]] const int nw_first =
+        min(nw, max((a.position + (min(row0 + 15, row_end - 1)) / a.group) / 32 + 1 - p0, 0));
     // Pages from which on some row of this wave masks keys (every row sees
     // the keys up to position + its first row's token; kPrepKeys' cached keys:
     // up to position - 1).  Keys before key_lo are masked too (kPrepKeys'
@@ -606,6 +609,27 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             });
         }
     };
+    // The last step of a wave whose first tile ends a page earlier (16 rows are
+    // at most 16 keys, so by one page at most): softmax and P.V of tile 1
+    // alone.  Tile 0's weights are 0 there, but a value that is not finite would
+    // still reach its rows (0 * inf is NaN).
+    auto step_second = [&](int i) __attribute__((always_inline)) {
+        if constexpr (NT == 2) {
+            const uint32_t vb = vring_lane + (i & 3) * PAGE_BYTES;
+            PV8 vf[DT];
+            static_for<0, DT>([&](auto dt) { lds_read<decltype(dt)::value * 1024>(vf[decltype(dt)::value], vb); });
+            static_for<0, 7>([&](auto part) { softmax(std::integral_constant<int, 1>{}, part, i); });
+            const PV8 hi = p_operand(ph[1]);
+            PV8 lo = hi;
+            if constexpr (PSPLIT) lo = p_operand(pl[1]);
+            static_for<0, DT>([&](auto dt) {
+                constexpr int d = decltype(dt)::value;
+                lds_wait<DT - 1 - d>(vf[d]);
+                acc[1][d] = mfma(vf[d], hi, acc[1][d]);
+                if constexpr (PSPLIT) acc[1][d] = mfma(vf[d], lo, acc[1][d]);
+            });
+        }
+    };
     auto step = [&](int i) __attribute__((always_inline)) {
         if constexpr (NT == 2) step_two(i);
         else step_one(i);
@@ -812,20 +836,41 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
+    auto meet = [&](int i) __attribute__((always_inline)) {
+        if ((i & 1) == 0) {
+            wait_vmcnt<0>();
+            prepare_v(i);
+            prepare_v(i + 1);
+            ring_barrier();
+            // Two groups read K one page further ahead.
+            if (i + KG + 2 < nl) stage(kh, i + KG + 2, kring);
+            if (i + KG + 3 < nl) stage(kh, i + KG + 3, kring);
+            if (i + 2 < nl) stage(vh, i + 2, vring);
+            if (i + 3 < nl) stage(vh, i + 3, vring);
+        }
+    };
+    auto mine = [&](int i) __attribute__((always_inline)) { return KG == 1 || (i & 1) == kg; };
     auto run_pages = [&]() __attribute__((always_inline)) {
-        for (int i = 0; i < nl; ++i) {
-            if ((i & 1) == 0) {
-                wait_vmcnt<0>();
-                prepare_v(i);
-                prepare_v(i + 1);
-                ring_barrier();
-                // Two groups read K one page further ahead.
-                if (i + KG + 2 < nl) stage(kh, i + KG + 2, kring);
-                if (i + KG + 3 < nl) stage(kh, i + KG + 3, kring);
-                if (i + 2 < nl) stage(vh, i + 2, vring);
-                if (i + 3 < nl) stage(vh, i + 3, vring);
+        if constexpr (NT == 2) {
+            // A wave whose first tile ends a page earlier leaves the loop at
+            // that page (2048 fp16 tokens of 32/8/128 at 6000: 247.0 us, 259.9
+            // with the branch in the loop, 245.9 without the step).
+            const int last = nw_first < nw && mine(nw - 1) ? nw - 1 : nl;
+            int i = 0;
+            for (; i < last; ++i) {
+                meet(i);
+                if (i < nw && mine(i)) step(i);
             }
-            if (i < nw && (KG == 1 || (i & 1) == kg)) step(i);
+            if (i < nl) {
+                meet(i);
+                step_second(i);
+                for (++i; i < nl; ++i) meet(i);
+            }
+        } else {
+            for (int i = 0; i < nl; ++i) {
+                meet(i);
+                if (i < nw && mine(i)) step(i);
+            }
         }
     };
     run_pages();

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import attention_ref as ref
+from redshift_amd import attention as A
 from redshift_amd.workloads import Workload, f32_to_bf16_bits, make_inputs, to_float
 from tests.test_attention_gpu import assert_parity, gpu_attention
 from tests.test_configs_gpu import PRECISE_REL_L2, precise_attention
@@ -79,3 +80,39 @@ def test_precise_two_passes_against_oracle(gpu, head_dim, tokens, position):
     want = ref.gqa_attention(q, k16, v16, position, w.scale)
     assert_parity(got, want)
     assert np.linalg.norm(got - want) / np.linalg.norm(want) <= PRECISE_REL_L2
+
+
+@pytest.mark.parametrize('bad', [float('inf'), float('nan')])
+@pytest.mark.parametrize('dtype', ['float16', 'bfloat16'])
+@pytest.mark.parametrize('kv,group,tokens,position', [(130, 1, 193, 16), (2, 8, 70, 333), (8, 4, 1540, 12)])
+def test_no_row_meets_values_past_its_own_tile(gpu, kv, group, tokens, position, dtype, bad):
+    """A value that is not finite reaches a row that does not see it only
+    through the 16-row tile that it shares a page walk with (its weight there
+    is 0): the two tiles of a wave stop at their own last pages.  Rows whose
+    tile ends before the bad key's page keep their bits (fp16), or stay within
+    the 16-bit weights' rounding (2^-8 of unit-variance values, bf16: such a
+    value sends its KV head to the exact products)."""
+    torch, d = gpu, 128
+    g = torch.Generator('cuda').manual_seed(tokens)
+    keys, dtype = position + tokens, getattr(torch, dtype)
+    cache = A.PagedKV(kv, d, A.round_capacity(keys), dtype)
+    k, v = (torch.randn(keys, kv, d, generator=g, device='cuda').to(dtype) for _ in 'kv')
+    q = torch.randn(tokens, kv * group, d, generator=g, device='cuda').to(dtype)
+    cache.pack(k, v)
+    want = A.attention(q, cache, position, d ** -.5).view(tokens, kv, group, d)
+    row = np.arange(tokens * group)
+    last = position + np.minimum(row // 16 * 16 + 15, row[-1]) // group      # the last key of the row's tile
+    pages = torch.from_numpy((last // 32 + 1).reshape(tokens, group)).cuda()
+    checked = 0
+    for key in sorted({*range((position + 31) // 32 * 32, keys, 32), keys - 1}):
+        hurt = v.clone()
+        hurt[key] = bad
+        cache.pack(k, hurt)
+        got = A.attention(q, cache, position, d ** -.5).view(tokens, kv, group, d)
+        clear = pages * 32 <= key
+        checked += int(clear.sum())
+        same = (got == want if dtype == torch.float16 else (got - want).abs() <= 2 ** -6).all(-1)
+        assert bool(same.permute(0, 2, 1)[clear].all()), key
+        # Every row that sees the key shows it.
+        assert not bool(torch.isfinite(got[key - position:].float()).any())
+    assert checked
