@@ -28,7 +28,8 @@
 // SIMD.  Online softmax in base 2 with a lazily moved row max (see ring.hip);
 // the scale is folded into the exponents' multiply-add, its sign applied to
 // the scores first where it is not positive, so any finite scale (zero and
-// negative ones included) gives the softmax of the scaled scores.  A page that
+// negative ones included) gives the softmax of the scaled scores as long as
+// these are finite in fp32 (kFoldMax below).  A page that
 // moves no row's max (nearly every page) needs neither the cross-lane row max
 // nor a rescaling factor: about 30 vector instructions and 8 exponentials per
 // page instead of 48 and 9 (bf16 2048 tokens at 6144: 330.3 -> 319.0 us; 3000
@@ -58,6 +59,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <climits>
 #include <type_traits>
 
 namespace rs {
@@ -366,9 +368,21 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // The scores are scaled by a positive factor in the exponents; a negative
     // or zero scale's sign is applied to the scores themselves.  A row's max
     // moves past move_above = (unscaled max) + kLazy / scale.
-    const float sign = a.scale_log2 > 0.f ? 1.f : a.scale_log2 < 0.f ? -1.f : 0.f;
-    const float scale = a.scale_log2 == 0.f ? 1.f : __builtin_fabsf(a.scale_log2);
-    const float lazy = kLazy / scale;
+    // A folded exponent, x * scale - (the rounded mx * scale), is not 0 at the
+    // max but off by that rounding, up to half a unit of the scaled max: a
+    // common factor of the row, which cancels while fp16 weights can hold it
+    // (to scaled maxima of about 2^27).  From kFoldMax on, far above the scores
+    // of ordinary data, the wave scales its scores before their max is taken
+    // (scale is then 1, and sign the whole scale): equal scores on both sides of
+    // the change get weights within 2^-13 * ln 2 of each other.
+    constexpr float kFoldMax = 4096.f;
+    auto uniform = [](float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); };
+    float sign = uniform(a.scale_log2 > 0.f ? 1.f : a.scale_log2 < 0.f ? -1.f : 0.f);
+    float scale = uniform(a.scale_log2 == 0.f ? 1.f : __builtin_fabsf(a.scale_log2));
+    float lazy = uniform(kLazy / scale);
+    // Scores that take a sign (or the whole scale) first do so where keys are
+    // masked: then on every page.
+    wave_first_limit = __builtin_amdgcn_readfirstlane(sign != 1.f ? INT_MIN : wave_first_limit);
     float move_above[NT], neg_mu[NT];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
@@ -424,7 +438,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             const int key0 = (p0 + i) * 32;
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = s[tt][j >> 2][j & 3];
-            if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo) || sign != 1.f) {
+            if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo)) {
                 keep_branch();
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -449,7 +463,10 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
                 const bool moved = mx > move_above[tt];
                 // `moved` implies a finite mx, so m - mx * scale is never
                 // -inf - (-inf).
-                const float to = mx * scale, alpha = moved ? __builtin_amdgcn_exp2f(m[tt] - to) : 1.f;
+                float to = mx * scale;
+                pin(to);   // rounded, as m holds it
+                float alpha = moved ? __builtin_amdgcn_exp2f(m[tt] - to) : 1.f;
+                pin(alpha);
                 m[tt] = moved ? to : m[tt];
                 move_above[tt] = moved ? mx + lazy : move_above[tt];
                 // The exponents' reference point: m, or 0 while the row has
@@ -459,6 +476,17 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
                 l[tt] *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) acc[tt][dt] *= alpha;
+                if (__any(__builtin_fabsf(neg_mu[tt]) >= kFoldMax) && scale != 1.f) {
+                    keep_branch();
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] *= scale;
+                    sign = a.scale_log2;
+                    scale = 1.f;
+                    lazy = kLazy;
+                    wave_first_limit = INT_MIN;
+#pragma unroll
+                    for (int t2 = 0; t2 < NT; ++t2) move_above[t2] = m[t2] + kLazy;
+                }
             }
             pin(neg_mu[tt]);
         } else if constexpr (part <= 3) {
@@ -891,7 +919,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             nl = max(0, (wg_keys + 31) / 32 - p0);
             nw = min(max((wave_keys + 31) / 32 - p0, 0), nl);
             limit[0] = a.position + row_token;
-            wave_first_limit = a.position + max(row0, 0) / a.group;
+            wave_first_limit = sign != 1.f ? INT_MIN : a.position + max(row0, 0) / a.group;
             key_lo = a.position;
             prep_new_keys();
             s[0][0] = s[0][1] = f32x4{0.f, 0.f, 0.f, 0.f};

@@ -48,6 +48,34 @@ def test_scales_against_oracle(gpu, head_dim, kv, group, tokens, position, scale
     assert_parity(gpu_attention(w, q, k, v, gpu, fill_nan=True, out_dtype=gpu.float32), want)
 
 
+@pytest.mark.parametrize('scale', [2.0 ** 3, 2.0 ** 13, -2.0 ** 20, 2.0 ** 60])
+@pytest.mark.parametrize('kind,head_dim,kv,group,tokens,position', [
+    ('f16', 128, 2, 8, 70, 333), ('bf16', 128, 2, 8, 70, 333), ('f16', 128, 130, 1, 193, 3),
+    ('bf16', 128, 130, 1, 193, 3), ('f16', 128, 2, 4, 40, 60), ('f16', 256, 2, 6, 70, 333),
+    ('bf16', 256, 2, 6, 40, 2000), ('precise', 128, 2, 4, 70, 333), ('precise', 256, 4, 6, 70, 1500),
+    ('precise', 256, 200, 1, 150, 40)])
+def test_scaled_scores_beyond_the_folded_exponents(gpu, kind, head_dim, kv, group, tokens, position, scale):
+    """Scaled scores that grow along the keys, past 2^12 (where a wave stops
+    folding the scale into its exponents) at the smallest scale and up to 2^74:
+    small integers times a power of two, so that the scores are exact and equal
+    ones have equal weights."""
+    w = Workload('large', kv * group, kv, head_dim, tokens, position, scale, 'f16', 5)
+    rng = np.random.default_rng(tokens)
+    keys = position + tokens
+    q = rng.integers(-2, 3, (tokens, kv * group, head_dim)).astype(np.float16)
+    k = (rng.integers(-1, 2, (keys, kv, head_dim)) * (1 + np.arange(keys) // 32 % 32)[:, None, None]).astype(np.float16)
+    v = rng.integers(-64, 65, k.shape).astype(np.float16) / 64
+    want = ref.gqa_attention(q, k, v, position, scale)
+    if kind == 'precise':
+        got = precise_attention(w, q.astype(np.float32), k, v, gpu)
+    else:
+        if kind == 'bf16':
+            w = Workload(**{**w.__dict__, 'dtype': 'bf16'})
+            q, k, v = (f32_to_bf16_bits(x.astype(np.float32)) for x in (q, k, v))
+        got = gpu_attention(w, q, k, v, gpu, out_dtype=gpu.float32)
+    assert_parity(got, want)
+
+
 @pytest.mark.parametrize('kv,group,tokens,position', [(2, 4, 70, 333), (130, 1, 193, 0)])
 def test_flagged_head_takes_the_exact_products(gpu, kv, group, tokens, position):
     """KV head 1's values lie far above the fp16 range (2^20 times N(0,1)):
