@@ -19,9 +19,12 @@ namespace {
 //      tokens of one key group (8 row accesses of 4 or 8 bytes, a wave
 //      covering whole row parts) and transposes them in registers.
 // Only tokens first .. first+count-1 are touched: other tokens' rows do not
-// exist, and their page slots keep their values (a V piece that holds such a
-// token is written value by value).  Buffers that are not 16-byte aligned
-// move value by value throughout.
+// exist, and their page slots keep their values (of a V piece that holds such
+// a token, four valid tokens are written at once, others value by value; a
+// loop of loads and stores over that page took one block up to 31 rounds: 31
+// tokens of 4 x 256 dims into pages 8.2 -> 3.9 us).  Buffers that are not
+// 16-byte aligned move value by value throughout, with kParts blocks per page
+// and head (31 tokens as above 7.1 -> 4.4 us against two batches in one block).
 // Rows taken into pages are loaded non-temporally (each is read once: 39.5 ->
 // 36.7 us); pages are loaded with the default policy (straight after their
 // writes they are partly cached: 29.1 against 40.4 us non-temporally).
@@ -35,6 +38,7 @@ struct ConvertArgs {
     bool whole;                           // 16-byte aligned buffers
 };
 constexpr int kConvertThreads = 256;
+constexpr int kParts = 8;   // blocks per (page, KV head) of buffers that are not aligned
 
 template <int D, bool TO_PAGES>
 __global__ __launch_bounds__(kConvertThreads)
@@ -42,11 +46,12 @@ void convert_pages(ConvertArgs a) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     constexpr int PAGE = 32 * D;
     const int sides = (a.pages[0] ? 1 : 0) + (a.pages[1] ? 1 : 0);
-    const size_t blocks = (size_t)a.n_pages * a.kv_heads * sides;
+    const size_t blocks = (size_t)a.n_pages * a.kv_heads * sides * (a.whole ? 1 : kParts);
     const size_t row_stride = (size_t)a.kv_heads * D;
     for (size_t b = blockIdx.x; b < blocks; b += gridDim.x) {
-        const int h = (int)(b % a.kv_heads);
-        const size_t ps = b / a.kv_heads;
+        const size_t ph = a.whole ? b : b / kParts;
+        const int h = (int)(ph % a.kv_heads);
+        const size_t ps = ph / a.kv_heads;
         const int side = sides == 2 ? (int)(ps % 2) : a.pages[0] ? 0 : 1;
         const int page = a.page0 + (int)(sides == 2 ? ps / 2 : ps);
         unsigned short *pg = a.pages[side] + (size_t)h * a.head_stride + (size_t)page * PAGE;
@@ -55,12 +60,26 @@ void convert_pages(ConvertArgs a) {
         unsigned short *rows = a.rows[side] + ((long long)page * 32 - a.first) * (long long)row_stride + (size_t)h * D;
         const int lo = max(a.first - page * 32, 0);                          // valid tokens of the page: lo .. hi-1
         const int hi = (int)min((long long)a.first + a.count - (long long)page * 32, 32LL);
-        if (!a.whole || (TO_PAGES && side == 1 && hi - lo < 32)) {
-            for (int e = lo * D + threadIdx.x; e < hi * D; e += kConvertThreads) {
-                const int p = e / D, d = e % D;
-                const size_t off = side ? v_page_offset(p, d, D) : k_page_offset(p, d, D);
-                if (TO_PAGES) pg[off] = rows[p * row_stride + d];
-                else rows[p * row_stride + d] = pg[off];
+        if (!a.whole) {
+            // Value by value, kValues in flight per thread (pages and rows may
+            // alias as far as the compiler knows, so it would wait for each).
+            constexpr int kValues = 32 / kParts * D / kConvertThreads;
+            const int p0 = (int)(b % kParts) * (32 / kParts), begin = max(lo, p0) * D;
+            const int end = min(hi, p0 + 32 / kParts) * D;
+            unsigned short v[kValues];
+            if (begin >= end) continue;
+#pragma unroll
+            for (int i = 0; i < kValues; ++i) {
+                const int e = min(begin + (int)threadIdx.x + i * kConvertThreads, end - 1), p = e / D, d = e % D;
+                v[i] = TO_PAGES ? rows[p * row_stride + d]
+                                : pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)];
+            }
+#pragma unroll
+            for (int i = 0; i < kValues; ++i) {
+                const int e = begin + threadIdx.x + i * kConvertThreads, p = e / D, d = e % D;
+                if (e >= end) continue;
+                if (TO_PAGES) pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)] = v[i];
+                else rows[p * row_stride + d] = v[i];
             }
         } else if (side == 0) {
             constexpr int PER = PAGE / 8 / kConvertThreads;
@@ -96,7 +115,7 @@ void convert_pages(ConvertArgs a) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int p = j / 4 * 16 + g * 4 + j % 4;   // slot j's token
-                VP *row = reinterpret_cast<VP *>(rows + p * row_stride + d);
+                VP *row = reinterpret_cast<VP *>(rows + (TO_PAGES ? min(max(p, lo), hi - 1) : p) * row_stride + d);
                 if constexpr (TO_PAGES) {
                     x[j] = __builtin_nontemporal_load(row);
                 } else {
@@ -106,11 +125,35 @@ void convert_pages(ConvertArgs a) {
                 }
             }
             if constexpr (TO_PAGES) {
+                if (hi - lo == 32) {
 #pragma unroll
-                for (int k = 0; k < VD; ++k) {
+                    for (int k = 0; k < VD; ++k) {
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) s[k][j] = x[j][k];
-                    *reinterpret_cast<V8 *>(slots + k * 8) = s[k];
+                        for (int j = 0; j < 8; ++j) s[k][j] = x[j][k];
+                        *reinterpret_cast<V8 *>(slots + k * 8) = s[k];
+                    }
+                } else {
+                    // Tokens outside lo .. hi-1 keep their slots, so what is
+                    // not theirs is not written: four tokens at once where all
+                    // of them are valid, else value by value.
+                    typedef unsigned short V4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        const int p0 = half * 16 + g * 4;
+                        const bool all = p0 >= lo && p0 + 4 <= hi;
+#pragma unroll
+                        for (int k = 0; k < VD; ++k) {
+                            unsigned short *dst = slots + k * 8 + half * 4;
+                            if (all) {
+                                *reinterpret_cast<V4 *>(dst) = V4{x[half * 4][k], x[half * 4 + 1][k],
+                                                                  x[half * 4 + 2][k], x[half * 4 + 3][k]};
+                            } else {
+#pragma unroll
+                                for (int j = 0; j < 4; ++j)
+                                    if (p0 + j >= lo && p0 + j < hi) dst[j] = x[half * 4 + j][k];
+                            }
+                        }
+                    }
                 }
             }
         }
@@ -139,7 +182,8 @@ void convert(void *k_pages, void *v_pages, const void *k_rows, const void *v_row
     a.count = count;
     a.page0 = first / kPageTokens;
     a.n_pages = (int)(((long long)first + count + kPageTokens - 1) / kPageTokens) - a.page0;
-    const size_t blocks = (size_t)a.n_pages * kv_heads * ((a.pages[0] != nullptr) + (a.pages[1] != nullptr));
+    const size_t blocks = (size_t)a.n_pages * kv_heads * ((a.pages[0] != nullptr) + (a.pages[1] != nullptr)) *
+                          (a.whole ? 1 : kParts);
     const void *kernel = head_dim == 256 ? (const void *)&convert_pages<256, TO_PAGES>
                                          : (const void *)&convert_pages<128, TO_PAGES>;
     void *args[] = {&a};

@@ -26,7 +26,8 @@ def _offset(torch, host, shift):
 @pytest.mark.parametrize('shift', [0, 1])
 @pytest.mark.parametrize('kv_heads,head_dim,capacity,first,count', [
     (4, 256, 32, 0, 32), (1, 128, 32, 31, 1), (4, 256, 96, 5, 70), (3, 128, 160, 32, 96),
-    (8, 128, 128, 17, 16), (2, 256, 2080, 0, 2049), (1, 256, 64, 40, 9)])
+    (8, 128, 128, 17, 16), (2, 256, 2080, 0, 2049), (1, 256, 64, 40, 9),
+    (1, 128, 32, 4, 4), (2, 256, 32, 1, 30), (3, 128, 64, 6, 50), (2, 256, 64, 19, 26)])
 def test_pack_and_unpack_bitwise(gpu, kv_heads, head_dim, capacity, first, count, shift, sides):
     torch, lib = gpu, library()
     rng = np.random.default_rng(first + count)
