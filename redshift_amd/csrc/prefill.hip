@@ -127,7 +127,9 @@ struct PrefillArgs {
     int flag_words;
     size_t head_stride;       // K and V pages
     int q_heads, kv_heads, group, rows, position, n_tiles;
-    float scale_log2;
+    // The score scale times log2(e), and what the kernel takes from it (scaled_by).
+    float scale_log2, scale_sign, scale_size, lazy;
+    int mask_from;       // INT_MAX; INT_MIN where the scores take the sign on every page
     // Key splits: workgroup (split, j, h) takes the split-th of `splits`
     // equal runs of the pages its rows see, and stores fp32 partials for the
     // combine kernel: its rows unnormalised ([kv_heads][splits][rows][D]),
@@ -376,13 +378,10 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // (scale is then 1, and sign the whole scale): equal scores on both sides of
     // the change get weights within 2^-13 * ln 2 of each other.
     constexpr float kFoldMax = 4096.f;
-    auto uniform = [](float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); };
-    float sign = uniform(a.scale_log2 > 0.f ? 1.f : a.scale_log2 < 0.f ? -1.f : 0.f);
-    float scale = uniform(a.scale_log2 == 0.f ? 1.f : __builtin_fabsf(a.scale_log2));
-    float lazy = uniform(kLazy / scale);
+    float sign = a.scale_sign, scale = a.scale_size, lazy = a.lazy;
     // Scores that take a sign (or the whole scale) first do so where keys are
     // masked: then on every page.
-    wave_first_limit = __builtin_amdgcn_readfirstlane(sign != 1.f ? INT_MIN : wave_first_limit);
+    wave_first_limit = min(wave_first_limit, a.mask_from);
     float move_above[NT], neg_mu[NT];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
@@ -919,7 +918,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             nl = max(0, (wg_keys + 31) / 32 - p0);
             nw = min(max((wave_keys + 31) / 32 - p0, 0), nl);
             limit[0] = a.position + row_token;
-            wave_first_limit = sign != 1.f ? INT_MIN : a.position + max(row0, 0) / a.group;
+            wave_first_limit = min(sign == a.scale_sign ? a.mask_from : INT_MIN, a.position + max(row0, 0) / a.group);
             key_lo = a.position;
             prep_new_keys();
             s[0][0] = s[0][1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1254,6 +1253,16 @@ size_t split_partial_bytes(const Shape &s, int splits) {
         : 0;
 }
 
+// The kernel's arguments for a score scale.  Worked out here: a division and
+// the selects cost a short call's prologue about 0.2 us.
+void scaled_by(PrefillArgs &a, float scale) {
+    a.scale_log2 = scale * 1.4426950408889634f;
+    a.scale_sign = a.scale_log2 > 0.f ? 1.f : a.scale_log2 < 0.f ? -1.f : 0.f;
+    a.scale_size = a.scale_log2 == 0.f ? 1.f : std::fabs(a.scale_log2);
+    a.lazy = kLazy / a.scale_size;
+    a.mask_from = a.scale_log2 > 0.f ? INT_MAX : INT_MIN;
+}
+
 }  // namespace
 
 PrefillPlan plan_prefill_for(const Shape &s, Dtype dtype, bool precise, int cus) {
@@ -1526,7 +1535,7 @@ void launch_prefill_prep(const FusedToken &tok, float *out, void *workspace, hip
     a.rows = s.group() * s.tokens;
     a.position = s.position;
     a.n_tiles = plan.row_wgs;
-    a.scale_log2 = (1.0f / 16.0f) * 1.4426950408889634f;
+    scaled_by(a, 1.0f / 16.0f);
     a.splits = plan.splits;
     a.key = tok.key;
     a.value = tok.value;
@@ -1562,7 +1571,7 @@ void launch_prefill_fused(const FusedToken &tok, float *out, void *workspace, hi
     a.rows = s.group() * s.tokens;
     a.position = s.position;
     a.n_tiles = plan.row_wgs;
-    a.scale_log2 = (1.0f / 16.0f) * 1.4426950408889634f;
+    scaled_by(a, 1.0f / 16.0f);
     a.splits = plan.splits;
     a.q_norm = tok.q_norm;
     a.k_norm = tok.k_norm;
@@ -1617,7 +1626,7 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
     const int rows = pairs ? kPairRows : plan.rows;
     const int row_wgs = (a.rows + rows - 1) / rows;
     a.n_tiles = row_wgs;
-    a.scale_log2 = scale * 1.4426950408889634f;
+    scaled_by(a, scale);
     a.splits = plan.splits;
     if (plan.splits > 1) {
         a.part_o = reinterpret_cast<float *>(static_cast<char *>(workspace) + plan.part_offset);
