@@ -182,14 +182,18 @@ size_t prefill_workspace_bytes(const Shape &s, Dtype dtype, bool precise);
 // rounds over the CUs than 1.5 times those of 192-row ones takes
 // kPreciseTwoPassRows rows per workgroup in two passes of its eight waves
 // (passes = 2): the later 128 rows first, then the earliest 64 rows, which
-// see the fewest keys, two waves on each 16-row tile.
-constexpr int kPrefillRows = 192, kPreciseRows = 128, kPreciseTwoPassRows = 192;
+// see the fewest keys, two waves on each 16-row tile.  A raw head_dim 128
+// call without key splits may launch workgroups of kPrefillPairRows rows
+// instead (pairs > 0), two 16-row tiles per wave, in one or two groups of four
+// waves; prefill.hip gives the rule with its measurements.
+constexpr int kPrefillRows = 192, kPreciseRows = 128, kPreciseTwoPassRows = 192, kPrefillPairRows = 128;
 constexpr int kPrefillMinSplitPages = 8, kPrefillMinSplitKeyPages = 32, kPrefillMaxSplits = 64;
 struct PrefillPlan {
     int rows;            // query rows per workgroup
     int row_wgs;         // workgroups of rows per KV head
     int splits;
     int passes;          // 1, or 2 (a precise call, eight waves over 192 rows)
+    int pairs;           // wave groups of the pair workgroups launched instead: 1 or 2, or 0 (none)
     size_t part_offset;  // split partials in the workspace
     size_t bytes;        // workspace
 };

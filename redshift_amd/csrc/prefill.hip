@@ -4,16 +4,17 @@
 // qvelox/server.py:187-191); this is the same causal GQA formula for long
 // token runs: row t sees keys 0..position+t.
 //
-// One workgroup owns 192 query rows (128 at head_dim 128, two tiles per wave:
-// kPairRows) of one KV head (row = token * group +
+// One workgroup owns 192 query rows of one KV head (row = token * group +
 // query head within the group) as twelve 16-row tiles, one per wave (three
-// per SIMD), whose query fragments stay in registers.  The tiles are dealt
-// out so that every SIMD has about the same number of (row, key) pairs (see
-// the kernel).  The workgroup walks the pages
-// that its last row can see through two rings of four LDS buffers, one for
-// K pages and one for V pages (16 KiB each at D=256), filled by direct
-// global->LDS loads two K and two V pages at every second step, a pair
-// ahead of the pair in use.  Since pages are stored in MFMA
+// per SIMD), whose query fragments stay in registers.  (Raw head_dim 128 calls
+// without key splits take 128 rows with two tiles per wave where that is
+// faster: prefill_pairs below.  A precise query takes 128 rows, or 192 in two
+// passes, on eight waves.)  The tiles are dealt out so that every SIMD has
+// about the same number of (row, key) pairs (see the kernel).  The workgroup
+// walks the pages that its last row can see through two rings of four LDS
+// buffers, one for K pages and one for V pages (16 KiB each at D=256), filled
+// by direct global->LDS loads two K and two V pages at every second step, a
+// pair ahead of the pair in use.  Since pages are stored in MFMA
 // operand order, every wave reads its A operands as conflict-free 16-byte
 // LDS fragments:
 //   S^T[key][row] = K[key][:] . Q[row][:]     (A = K tile from LDS, B = Q)
@@ -1121,29 +1122,53 @@ void attention_prefill_bf16(PrefillArgs a) {
 // (attention_prefill_2pass) when that saves rounds of workgroups.
 
 // Raw head_dim 128 calls without key splits have two more instances, of
-// kPairRows = 128 rows per workgroup, two 16-row tiles in each of four waves
-// (step_two).  All three reach about the same rate on a full device (3072
-// fp16 tokens of 32/8/128 at 20,000: 1060 us, 1.02 PFLOP/s, in two rounds of
-// 192-row workgroups or three of 128-row pairs); what differs is how well
-// their workgroups fill it.
+// kPrefillPairRows = 128 rows per workgroup, two 16-row tiles in each of four
+// waves (step_two).  All reach about the same rate on a full device; what
+// differs is how well their workgroups fill it.  Below, fp16, times in us in a
+// graph, 256 CUs.
 //   192 rows, twelve waves: the serpentine deal gives every workgroup the same
 //     work, but a round of workgroups that is not full is lost whole.  Taken
-//     for one round at most (1100 tokens at 3000: 91.2 against 104.9 us with
-//     pairs; 1500 at 0: 32.1 against 39.3).
-//   Pairs, four waves (216 VGPRs, 64 KiB of rings: two workgroups per CU):
+//     for one round at most (1500 tokens of 32/8/128 at 0: 32.1, with pairs
+//     39.3).
+//   Pairs, four waves (216 VGPRs, 64 KiB of rings: two workgroups per CU): for
 //     several rounds, the longest workgroups first and the CUs refilled as
-//     they end (2048 at 30,000: 999 us, 192-row workgroups 1581; 3000 at
-//     0: 83.1 against 107.8; 1600 at 3000: 120.6 against 176.3).
+//     they end (2048 of 32/8/128 at 30,000: 999, 192-row workgroups 1581; 3000
+//     at 0: 83.1 and 107.8).  Two workgroups of a CU take about 5/4, and one
+//     alone about as long, as a round of 192-row ones, so counting both in
+//     quarter rounds tells which needs fewer: 130 tokens of 387/129/128 at 2000
+//     (387 against 516 workgroups) 96.8 in 192 rows, 116.7 in pairs; 390 of
+//     129/129/128 at 2000 105.8 and 119.3.  On a prefix shorter than three times
+//     the chunk the causal tail decides instead: pairs win by up to a third (130
+//     of 387/129/128 at 0: 16.9 and 14.1; 2750 of 32/8/128 at 0: 96.1 and 74.5)
+//     or come within 5% (2750 at 2750: 212.0 and 222.6, at 5500 336.9 and 337.9).
 //   Pairs in two groups of four waves, on the even and the odd pages (KG = 2):
-//     where every 128-row workgroup has a CU of its own, four waves alone
-//     would leave it half empty (1000 at 3000: 72.3 us, 89.5 with four waves,
-//     83.5 with the 192-row workgroups).  A prefix shorter than a quarter of
-//     the chunk keeps the 192-row deal, since the last rows' workgroup, with
-//     its many keys, then sets the time (1000 at 200: 28.1 and 28.0 us; 1000
-//     at 0: 25.1 against 24.1; 4000 of 8/2/128 at 0: 70.1 against 66.2).
+//     where every 128-row workgroup has a CU of its own, four waves alone would
+//     leave it half empty (1000 at 3000: 72.3, 89.5 with four waves, 83.5 with
+//     the 192-row workgroups).  They pay where the 192-row deal has three waves
+//     on a SIMD; with one or two (few rows per head) its steps are shorter than
+//     the pairs' and the merge is not paid back (16 tokens of 32/8/128 at 200:
+//     8.1 in 192 rows, 9.9 in pairs; 64 at 200 10.6 and 12.6; 64 of 129/129/128 at
+//     2000 43.7 and 46.0).  Nor is it on few pages, or where the last rows'
+//     workgroup, with its many keys, sets the time: from 256 cached tokens and
+//     two fifths of the chunk on pairs are 0.99 to 1.16 times as fast (200 tokens
+//     of 32/8/128 at 200: 14.3 and 15.0, at 300 16.6 and 16.2; 500 at 128: 17.9
+//     and 18.3, at 300 21.1 and 21.3; 1000 at 600 35.1 and 34.3; 2244 of 12/1/128
+//     at 1022 63.9 and 61.1).
 // Calls with key splits run few pages per workgroup and keep twelve waves (500
 // bf16 tokens of 8/2/128 at 5000: 29.6 against 32.5 us with pairs).
-constexpr int kPairRows = 128;
+int prefill_pairs(const Shape &s, int row_wgs, int cus) {
+    const long long rows = (long long)s.group() * s.tokens;
+    const long long wide = (long long)row_wgs * s.kv_heads;   // 192-row workgroups
+    const long long paired = (rows + kPrefillPairRows - 1) / kPrefillPairRows * s.kv_heads;
+    if (wide > cus) {
+        const long long rest = paired % (2LL * cus);
+        const long long wide_quarters = 4 * ((wide + cus - 1) / cus);
+        const long long paired_quarters = 5 * (paired / (2LL * cus)) + (rest == 0 ? 0 : rest <= cus ? 4 : 5);
+        return paired_quarters <= wide_quarters || s.position < 3LL * s.tokens ? 1 : 0;
+    }
+    const long long tiles = ((rows + 15) / 16 + row_wgs - 1) / row_wgs;   // of the fullest 192-row workgroup
+    return paired <= cus && tiles > 8 && s.position >= 256 && 5LL * s.position >= 2LL * s.tokens ? 2 : 0;
+}
 
 // The raw instances: fp16 pages; bf16 pages, V through the conversion pass
 // below (attention_prefill_bf16).
@@ -1276,6 +1301,7 @@ PrefillPlan plan_prefill_for(const Shape &s, Dtype dtype, bool precise, int cus)
         p.splits = (int)std::max(1LL, std::min<long long>({cus / base, pages / kPrefillMinSplitPages,
                                                            kPrefillMaxSplits}));
     p.passes = 1;
+    p.pairs = !precise && s.head_dim == 128 && p.splits == 1 ? prefill_pairs(s, p.row_wgs, cus) : 0;
     if (precise && p.splits == 1) {
         const long long rows = (long long)s.group() * s.tokens;
         const long long wgs2 = (rows + kPreciseTwoPassRows - 1) / kPreciseTwoPassRows;
@@ -1501,6 +1527,7 @@ PrefillPlan plan_prefill_prep_for(int tokens, int position, int cus) {
     p.rows = kPreciseRows;
     p.row_wgs = (s.group() * tokens + p.rows - 1) / p.rows;
     p.passes = 1;
+    p.pairs = 0;
     // Runs over the cached pages as plan_prefill_for splits a call's pages
     // (the last run, the shortest, also takes the chunk's keys).
     const long long cached = ((long long)position + kPageTokens - 1) / kPageTokens;
@@ -1617,14 +1644,8 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
     a.rows = s.group() * s.tokens;
     a.position = s.position;
     const bool d256 = s.head_dim == 256;
-    // See kPairRows.
-    const int cus = device_cu_count();
-    const bool may_pair = !precise && !d256 && plan.splits == 1;
-    const long long pair_wgs = (a.rows + (long long)kPairRows - 1) / kPairRows * s.kv_heads;
-    const bool groups = may_pair && pair_wgs <= cus && 4LL * s.position >= s.tokens;
-    const bool pairs = groups || (may_pair && (long long)plan.row_wgs * s.kv_heads > cus);
-    const int rows = pairs ? kPairRows : plan.rows;
-    const int row_wgs = (a.rows + rows - 1) / rows;
+    const int rows = plan.pairs ? kPrefillPairRows : plan.rows;
+    const int row_wgs = plan.pairs ? (a.rows + rows - 1) / rows : plan.row_wgs;
     a.n_tiles = row_wgs;
     scaled_by(a, scale);
     a.splits = plan.splits;
@@ -1634,7 +1655,7 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
         // Raw rows that combine_prefill merges travel as 16-bit planes.
         a.half_parts = !precise && plan.splits <= kCombineWideBatch;
     }
-    const int threads = (pairs ? (groups ? 8 : 4) : plan.passes == 2 ? 8 : rows / 16) * kWave;
+    const int threads = (plan.pairs ? 4 * plan.pairs : plan.passes == 2 ? 8 : rows / 16) * kWave;
     const long long grid = (long long)row_wgs * s.kv_heads * plan.splits;
     require(grid * threads < (1LL << 32), "prefill launch exceeds 2^32 work-items");
     void *args[] = {&a};
@@ -1669,10 +1690,10 @@ void launch_prefill(const Shape &s, Dtype dtype, bool precise, float scale, cons
         a.v_flags = flags;
         a.flag_words = c.pages;
     }
-    const void *kernel = d256     ? prefill_kernel<256, kPrefillRows, 1, 1>(dtype, out_f32)
-                         : !pairs ? prefill_kernel<128, kPrefillRows, 1, 1>(dtype, out_f32)
-                         : groups ? prefill_kernel<128, kPairRows, 2, 2>(dtype, out_f32)
-                                  : prefill_kernel<128, kPairRows, 2, 1>(dtype, out_f32);
+    const void *kernel = d256              ? prefill_kernel<256, kPrefillRows, 1, 1>(dtype, out_f32)
+                         : plan.pairs == 0 ? prefill_kernel<128, kPrefillRows, 1, 1>(dtype, out_f32)
+                         : plan.pairs == 1 ? prefill_kernel<128, kPrefillPairRows, 2, 1>(dtype, out_f32)
+                                           : prefill_kernel<128, kPrefillPairRows, 2, 2>(dtype, out_f32);
     check(hipLaunchKernel(kernel, dim3((unsigned)grid), dim3(threads), args, 0, stream));
     combine();
 }

@@ -338,6 +338,52 @@ void prefill_planner_sweep() {
     std::printf("abi_sanitize: %d prefill plans checked\n", plans);
 }
 
+// Which raw head_dim 128 calls launch pair workgroups (PrefillPlan::pairs): the
+// measured sides of every line on 256 CUs, and on the sweep's shapes and
+// devices the launch's own limits and the rule's cases.
+void prefill_pairs_sweep() {
+    struct Case { int q_heads, kv_heads, head_dim, tokens, position, pairs; };
+    const Case measured[] = {
+        // One round of 192-row workgroups: two groups only with three waves
+        // per SIMD, 256 cached tokens and two fifths of the chunk.
+        {32, 8, 128, 16, 200, 0}, {32, 8, 128, 64, 200, 0}, {32, 8, 128, 64, 900, 0}, {28, 4, 128, 32, 700, 0},
+        {8, 2, 128, 64, 700, 0}, {16, 16, 128, 128, 400, 0}, {129, 129, 128, 64, 2000, 0}, {200, 200, 128, 100, 500, 0},
+        {32, 8, 128, 200, 200, 0}, {32, 8, 128, 128, 200, 0}, {32, 8, 128, 500, 128, 0}, {32, 8, 128, 200, 300, 2},
+        {32, 8, 128, 500, 400, 2}, {32, 8, 128, 900, 700, 2}, {32, 8, 128, 1000, 300, 0}, {32, 8, 128, 1000, 3000, 2},
+        {12, 1, 128, 16, 700, 2}, {12, 1, 128, 2244, 1022, 2}, {28, 4, 128, 64, 600, 2}, {32, 8, 128, 1500, 0, 0}, {32, 8, 128, 1100, 3000, 0},
+        // Several rounds: pairs, unless they take more of them on a long prefix.
+        {32, 8, 128, 3000, 0, 1}, {32, 8, 128, 2048, 30000, 1}, {32, 8, 128, 1600, 3000, 1}, {32, 8, 128, 3100, 24000, 1},
+        {387, 129, 128, 130, 0, 1}, {387, 129, 128, 130, 2000, 0}, {129, 129, 128, 390, 2000, 0},
+        {129, 129, 128, 193, 2000, 1}, {32, 8, 128, 2750, 5500, 1}, {32, 8, 128, 2750, 22000, 0},
+        // Key splits, 256-dim calls.
+        {8, 2, 128, 500, 5000, 0}, {24, 4, 256, 2048, 6144, 0}, {24, 4, 256, 4096, 0, 0}};
+    for (const Case &c : measured)
+        for (int dt = 0; dt < 2; ++dt) {
+            const rs::Shape s{c.q_heads, c.kv_heads, c.head_dim, c.tokens, c.position, 0};
+            EXPECT(rs::plan_prefill_for(s, dt ? rs::Dtype::BF16 : rs::Dtype::F16, false, 256).pairs == c.pairs);
+            EXPECT(rs::plan_prefill_for(s, rs::Dtype::F16, true, 256).pairs == 0);
+        }
+    int plans = 0;
+    for (int hkv : {1, 2, 8, 64, 129, 256})
+        for (int group : {1, 3, 4, 8, 48})
+            for (int cus : {1, 8, 80, 256, 304})
+                for (int pos : {0, 31, 255, 256, 300, 1000, 6144, 139263, 1 << 30})
+                    for (int tokens : {49, 64, 130, 193, 600, 2048, 8192, 1 << 20}) {
+                        if ((long long)hkv * group * tokens > (1LL << 28) || group * tokens <= rs::kMaxRows) continue;
+                        const rs::Shape s{hkv * group, hkv, 128, tokens, pos, 0};
+                        const rs::PrefillPlan p = rs::plan_prefill_for(s, rs::Dtype::F16, false, cus);
+                        ++plans;
+                        const long long R = (long long)group * tokens;
+                        const long long pair_wgs = (R + rs::kPrefillPairRows - 1) / rs::kPrefillPairRows * hkv;
+                        EXPECT(p.pairs >= 0 && p.pairs <= 2 && (p.pairs == 0 || p.splits == 1));
+                        if (p.pairs) EXPECT(pair_wgs * p.pairs * 256 < (1LL << 32));
+                        if (p.pairs == 2) EXPECT(pair_wgs <= cus && pos >= 256 && 5LL * pos >= 2LL * tokens);
+                        if ((long long)p.row_wgs * hkv <= cus) EXPECT(p.pairs != 1);
+                        else EXPECT(p.pairs == 1 || pos >= 3LL * tokens);
+                    }
+    std::printf("abi_sanitize: %d pair choices checked\n", plans);
+}
+
 // The prepared prefill of a fused chunk (plan_prefill_prep_for): chunks of
 // 9 .. 128 - position % 32 tokens fit; 128-row workgroups; runs over the
 // cached pages as plan_prefill_for splits a call's pages (one below
@@ -567,6 +613,7 @@ int main(int argc, char **argv) {
     device_entry_validation();
     planner_sweep();
     prefill_planner_sweep();
+    prefill_pairs_sweep();
     prefill_prep_planner_sweep();
     int devices = 0;
     const bool gpu = hipGetDeviceCount(&devices) == hipSuccess && devices > 0;

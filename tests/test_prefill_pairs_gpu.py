@@ -2,9 +2,10 @@
 16-row tiles per wave; two wave groups over alternate pages where every
 workgroup has a CU of its own) and the second pass of the two-pass precise
 prefill, against the oracle at the sizes where they can go wrong: a last wave
-with one row, with one tile or with all but one row; one page (the second
-group has none), two and odd page counts; a row max that moves late (outlier
-keys); negative and zero scales; bf16 pages, a flagged KV head among them (the
+with one row, with one tile or with all but one row; even and odd page counts
+(for the second pass also one page, of which the second group has none), and
+calls on both sides of each line of their dispatch; a row max that moves late
+(outlier keys); negative and zero scales; bf16 pages, a flagged KV head among them (the
 exact products); stale slots past the last key hold NaN.  Bounds: max-abs
 2e-3, relative L2 1e-3 on the fp32 output, as for the other raw calls."""
 import numpy as np
@@ -19,17 +20,20 @@ from tests.test_configs_gpu import PRECISE_REL_L2, precise_attention
 pytestmark = pytest.mark.gpu
 
 
-# kv_heads, group, tokens, position.  Up to 256 workgroups of 128 rows after a
-# prefix (two wave groups on 256 CUs); more than 256 workgroups of 192 rows (one
-# group, two workgroups a CU); one round of 192-row workgroups.
-GROUPS = [(1, 8, 7, 2), (2, 7, 7, 25), (1, 4, 13, 20), (2, 4, 33, 31), (1, 1, 159, 40), (1, 5, 200, 700),
-          (3, 8, 70, 900)]
+# kv_heads, group, tokens, position, on 256 CUs.  FEW: few rows or pages per
+# head (192-row workgroups).  GROUPS: two wave groups, from 256 cached tokens on.
+# SINGLE: more than 256 workgroups of 192 rows (one group, two workgroups a CU).
+# ROUND: one round of 192-row workgroups.  LONG: several rounds, fewer of 192
+# rows, on a long prefix.
+FEW = [(1, 8, 7, 2), (2, 7, 7, 25), (1, 4, 13, 20), (2, 4, 33, 31), (1, 1, 159, 40)]
+GROUPS = [(1, 5, 200, 700), (3, 8, 70, 900), (1, 1, 129, 256), (1, 1, 161, 263), (1, 12, 13, 260), (1, 4, 130, 330)]
 SINGLE = [(8, 4, 1540, 5), (130, 1, 193, 0), (130, 1, 257, 40), (65, 2, 400, 600)]
 ROUND = [(1, 1, 159, 1), (8, 4, 200, 0)]
+LONG = [(129, 3, 130, 400)]
 
 
 @pytest.mark.parametrize('dtype', ['f16', 'bf16'])
-@pytest.mark.parametrize('kv,group,tokens,position', GROUPS + SINGLE + ROUND)
+@pytest.mark.parametrize('kv,group,tokens,position', FEW + GROUPS + SINGLE + ROUND + LONG)
 def test_pairs_against_oracle(gpu, kv, group, tokens, position, dtype):
     w = Workload('pairs', kv * group, kv, 128, tokens, position, 1 / 128 ** .5, dtype, tokens, 1.0, 0.5,
                  min(8, tokens + position), 8.0)
