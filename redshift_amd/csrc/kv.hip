@@ -23,8 +23,8 @@ namespace {
 // a token, four valid tokens are written at once, others value by value; a
 // loop of loads and stores over that page took one block up to 31 rounds: 31
 // tokens of 4 x 256 dims into pages 8.2 -> 3.9 us).  Buffers that are not
-// 16-byte aligned move value by value throughout, with kParts blocks per page
-// and head (31 tokens as above 7.1 -> 4.4 us against two batches in one block).
+// 16-byte aligned move value by value throughout, four values in flight per
+// thread, in eight blocks per page and head where the pages alone are few.
 // Rows taken into pages are loaded non-temporally (each is read once: 39.5 ->
 // 36.7 us); pages are loaded with the default policy (straight after their
 // writes they are partly cached: 29.1 against 40.4 us non-temporally).
@@ -36,9 +36,13 @@ struct ConvertArgs {
     size_t head_stride;
     int kv_heads, first, count, page0, n_pages;
     bool whole;                           // 16-byte aligned buffers
+    int parts;                            // blocks per (page, KV head, K or V): 1 or, unaligned, 8
 };
 constexpr int kConvertThreads = 256;
-constexpr int kParts = 8;   // blocks per (page, KV head) of buffers that are not aligned
+// Unaligned buffers: eight blocks per (page, KV head, K or V) where these are
+// fewer than the CUs (1000 tokens of 8 x 128 dims, 512 pages and heads: 9.9 us in
+// eight blocks each).
+constexpr int kConvertBlocks = 256;
 
 template <int D, bool TO_PAGES>
 __global__ __launch_bounds__(kConvertThreads)
@@ -46,10 +50,10 @@ void convert_pages(ConvertArgs a) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     constexpr int PAGE = 32 * D;
     const int sides = (a.pages[0] ? 1 : 0) + (a.pages[1] ? 1 : 0);
-    const size_t blocks = (size_t)a.n_pages * a.kv_heads * sides * (a.whole ? 1 : kParts);
+    const size_t blocks = (size_t)a.n_pages * a.kv_heads * sides * a.parts;
     const size_t row_stride = (size_t)a.kv_heads * D;
     for (size_t b = blockIdx.x; b < blocks; b += gridDim.x) {
-        const size_t ph = a.whole ? b : b / kParts;
+        const size_t ph = b / a.parts;
         const int h = (int)(ph % a.kv_heads);
         const size_t ps = ph / a.kv_heads;
         const int side = sides == 2 ? (int)(ps % 2) : a.pages[0] ? 0 : 1;
@@ -61,25 +65,25 @@ void convert_pages(ConvertArgs a) {
         const int lo = max(a.first - page * 32, 0);                          // valid tokens of the page: lo .. hi-1
         const int hi = (int)min((long long)a.first + a.count - (long long)page * 32, 32LL);
         if (!a.whole) {
-            // Value by value, kValues in flight per thread (pages and rows may
+            // Value by value, kBatch in flight per thread (pages and rows may
             // alias as far as the compiler knows, so it would wait for each).
-            constexpr int kValues = 32 / kParts * D / kConvertThreads;
-            const int p0 = (int)(b % kParts) * (32 / kParts), begin = max(lo, p0) * D;
-            const int end = min(hi, p0 + 32 / kParts) * D;
-            unsigned short v[kValues];
-            if (begin >= end) continue;
+            constexpr int kBatch = 4;
+            const int p0 = (int)(b % a.parts) * (32 / a.parts), end = min(hi, p0 + 32 / a.parts) * D;
+            for (int e0 = max(lo, p0) * D + threadIdx.x; e0 < end; e0 += kBatch * kConvertThreads) {
+                unsigned short v[kBatch];
 #pragma unroll
-            for (int i = 0; i < kValues; ++i) {
-                const int e = min(begin + (int)threadIdx.x + i * kConvertThreads, end - 1), p = e / D, d = e % D;
-                v[i] = TO_PAGES ? rows[p * row_stride + d]
-                                : pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)];
-            }
+                for (int i = 0; i < kBatch; ++i) {
+                    const int e = min(e0 + i * kConvertThreads, end - 1), p = e / D, d = e % D;
+                    v[i] = TO_PAGES ? rows[p * row_stride + d]
+                                    : pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)];
+                }
 #pragma unroll
-            for (int i = 0; i < kValues; ++i) {
-                const int e = begin + threadIdx.x + i * kConvertThreads, p = e / D, d = e % D;
-                if (e >= end) continue;
-                if (TO_PAGES) pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)] = v[i];
-                else rows[p * row_stride + d] = v[i];
+                for (int i = 0; i < kBatch; ++i) {
+                    const int e = e0 + i * kConvertThreads, p = e / D, d = e % D;
+                    if (e >= end) break;
+                    if (TO_PAGES) pg[side ? v_page_offset(p, d, D) : k_page_offset(p, d, D)] = v[i];
+                    else rows[p * row_stride + d] = v[i];
+                }
             }
         } else if (side == 0) {
             constexpr int PER = PAGE / 8 / kConvertThreads;
@@ -182,12 +186,12 @@ void convert(void *k_pages, void *v_pages, const void *k_rows, const void *v_row
     a.count = count;
     a.page0 = first / kPageTokens;
     a.n_pages = (int)(((long long)first + count + kPageTokens - 1) / kPageTokens) - a.page0;
-    const size_t blocks = (size_t)a.n_pages * kv_heads * ((a.pages[0] != nullptr) + (a.pages[1] != nullptr)) *
-                          (a.whole ? 1 : kParts);
+    const size_t blocks = (size_t)a.n_pages * kv_heads * ((a.pages[0] != nullptr) + (a.pages[1] != nullptr));
+    a.parts = a.whole || blocks >= kConvertBlocks ? 1 : 8;
     const void *kernel = head_dim == 256 ? (const void *)&convert_pages<256, TO_PAGES>
                                          : (const void *)&convert_pages<128, TO_PAGES>;
     void *args[] = {&a};
-    check(hipLaunchKernel(kernel, dim3((unsigned)std::min<size_t>(blocks, 1u << 20)), dim3(kConvertThreads), args, 0,
+    check(hipLaunchKernel(kernel, dim3((unsigned)std::min<size_t>(blocks * a.parts, 1u << 20)), dim3(kConvertThreads), args, 0,
                           stream));
 }
 
