@@ -271,7 +271,8 @@ def provenance(torch, lib_path):
     card = gpu_card(torch)
     lib_sha = sha256_of([Path(lib_path)])
     head, head_from = commit_of(lib_sha)
-    return {'library_sha256': lib_sha, 'sources_sha256': sha256_of(sources),
+    return {'library_sha256': lib_sha, 'front_sha256': sha256_of([Path(lib_path).with_name('redshift_front.so')]),
+            'sources_sha256': sha256_of(sources),
             'sources': 'redshift_amd/csrc/*, include/*.h, redshift_amd/*.py, bench.py',
             'git_head': head, 'git_head_from': head_from, 'device': props.name, 'arch': props.gcnArchName,
             'cus': props.multi_processor_count, 'torch': torch.__version__,

@@ -9,28 +9,55 @@ the others and raises every error of the checks.
 import ctypes as ct
 import importlib.machinery
 import importlib.util
+import json
 import math
-from pathlib import Path
+import warnings
 
 import torch
 
-from .runtime import QV_BF16, QV_F16, QV_F32, check, library
+from .build import BUILD_INFO, FRONT_LIBRARY, file_sha256, front_target
+from .runtime import DEFAULT_LIBRARY, QV_BF16, QV_F16, QV_F32, check, library
 
 PAGE_TOKENS = 32
 # Query rows (group * tokens) per KV head that one split/combine pair serves.
 MAX_CHUNK_ROWS = 48
 
-
-FRONT_LIBRARY = Path(__file__).resolve().parent / 'lib' / 'redshift_front.so'
 _FRONT = None
 
 
+class _PythonRoute:
+    """Stands in for the native calls: takes none."""
+    attention = attention_fused = staticmethod(lambda *args: None)
+
+
+def _front_mismatch():
+    """Why the native calls beside the library cannot be used, or None: they
+    must be those of the library's own build, for this torch and Python."""
+    try:
+        info = json.loads(BUILD_INFO.read_text())
+        library_sha256, front_sha256 = file_sha256(DEFAULT_LIBRARY), file_sha256(FRONT_LIBRARY)
+    except (OSError, ValueError) as error:
+        return str(error)
+    if (info.get('library_sha256'), info.get('front_sha256')) != (library_sha256, front_sha256):
+        return f'{FRONT_LIBRARY} and {DEFAULT_LIBRARY} are not from one build'
+    for name, value in front_target(torch).items():
+        if info.get(name) != value:
+            return f'{FRONT_LIBRARY} was built for {name} {info.get(name)}, not {value}'
+    return None
+
+
 def _load_front():
-    """The native calls, bound to the process-wide library (on first use)."""
+    """The native calls, bound to the process-wide library (on first use).
+    Without them every call takes the Python route, which launches the same
+    kernels after more time on the host."""
     global _FRONT
     lib = library()
-    if not FRONT_LIBRARY.exists():
-        raise RuntimeError(f'{FRONT_LIBRARY} is missing: build it with `python -m redshift_amd.build`')
+    mismatch = _front_mismatch()
+    if mismatch:
+        warnings.warn(f'no native calls ({mismatch}): attention() and attention_fused() run from Python; '
+                      'build them with `python -m redshift_amd.build`', RuntimeWarning, stacklevel=3)
+        _FRONT = _PythonRoute
+        return _FRONT
     loader = importlib.machinery.ExtensionFileLoader('redshift_front', str(FRONT_LIBRARY))
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader('redshift_front', loader))
     loader.exec_module(module)

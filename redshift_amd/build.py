@@ -2,7 +2,10 @@
 
 Usage: ``python -m redshift_amd.build`` (or ``__graft_entry__.build()``).
 Objects go to ``redshift_amd/_build/``, the library to
-``redshift_amd/lib/libredshift_hip.so``.  Every call recompiles.
+``redshift_amd/lib/libredshift_hip.so``.  Every call recompiles.  The library
+needs hipcc alone; the torch front end's native calls beside it also need torch,
+a host compiler and Python's headers, and are left out where these are missing
+(attention.py then makes the same calls from Python).
 """
 import hashlib
 import json
@@ -26,9 +29,10 @@ PROBE_LIBRARY = PACKAGE / 'lib' / 'libredshift_probe.so'
 # headers; attention.py loads it beside the library, which knows no torch).
 FRONT_SOURCE = PACKAGE / 'csrc' / 'front.cpp'
 FRONT_LIBRARY = PACKAGE / 'lib' / 'redshift_front.so'
-# The commit the library was built from and the library's SHA-256, written
-# beside it by build(), for trees copied without their .git (bench.py's
-# provenance).
+# Written beside them by build(): the commit they were built from and the
+# library's SHA-256, for trees copied without their .git (bench.py's
+# provenance), and the front end's SHA-256 with the torch and Python it was
+# compiled for (attention.py loads no other).
 BUILD_INFO = PACKAGE / 'lib' / 'build_info.json'
 ARCH = 'gfx950'
 # The host-sanitizer gate: the library's sources and a driver over its C ABI,
@@ -141,42 +145,67 @@ def _link(objects, library):
     library.parent.mkdir(exist_ok=True)
     tmp = library.with_suffix('.so.tmp')
     _run([hipcc(), '-shared', '-fPIC', f'--offload-arch={ARCH}', *[str(o) for o in objects], '-o', str(tmp)])
-    os.replace(tmp, library)
+    return tmp
 
 
 def build_front():
-    """Compile the torch front end's extension (host code only)."""
-    import torch
-    base = Path(torch.__file__).resolve().parent
+    """Compile the torch front end's extension (host code only) to a temporary
+    file; returns its path and what it was compiled for, or None and the
+    reason where something that it needs is missing."""
+    try:
+        import torch
+    except ImportError:
+        return None, 'torch is not importable'
+    base, headers = Path(torch.__file__).resolve().parent, sysconfig.get_paths()['include']
     compiler = shutil.which('g++') or shutil.which('c++')
     if compiler is None:
-        raise RuntimeError('g++ not found: a host compiler is required to build the torch front end')
+        return None, 'there is no host compiler (g++)'
+    if not (Path(headers) / 'Python.h').exists():
+        return None, 'Python.h is not installed'
     FRONT_LIBRARY.parent.mkdir(exist_ok=True)
     tmp = FRONT_LIBRARY.with_suffix('.so.tmp')
-    stderr = _run([compiler, '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall',
-                   f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
-                   f'-I{sysconfig.get_paths()["include"]}', f'-I{base / "include"}',
-                   f'-I{base / "include" / "torch" / "csrc" / "api" / "include"}',
-                   str(FRONT_SOURCE), '-o', str(tmp), f'-L{base / "lib"}', '-lc10', '-ltorch_cpu', '-ltorch_python'])
-    os.replace(tmp, FRONT_LIBRARY)
-    return stderr
+    _run([compiler, '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall',
+          f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+          f'-I{headers}', f'-I{ROOT / "include"}', f'-I{base / "include"}',
+          f'-I{base / "include" / "torch" / "csrc" / "api" / "include"}',
+          str(FRONT_SOURCE), '-o', str(tmp), f'-L{base / "lib"}', '-lc10', '-ltorch_cpu', '-ltorch_python'])
+    return tmp, front_target(torch)
+
+
+def front_target(torch):
+    """What the front end is compiled for."""
+    return {'torch': str(torch.__version__), 'python': sysconfig.get_config_var('SOABI')}
+
+
+def file_sha256(path):
+    return hashlib.sha256(Path(path).read_bytes()).hexdigest()
 
 
 def build(verbose=False, jobs=None):
     """Compile every source and link the shared library (and the probe
-    library and the torch front end beside it); returns the attention
-    library's path."""
+    library and, where it can be built, the torch front end beside it);
+    returns the attention library's path.  The front end of an earlier build
+    never stays beside a newer library, and BUILD_INFO describes what is there
+    even if the front end does not compile, which is an error."""
     names = SOURCES + PROBE_SOURCES
     results = _compile_all(PACKAGE / '_build', [(name, PACKAGE / 'csrc' / name) for name in names], [], jobs)
     for _, stderr in results:
         if verbose and stderr:
             print(stderr, file=sys.stderr)
     objects = dict(zip(names, (o for o, _ in results)))
-    _link([objects[name] for name in SOURCES], LIBRARY)
-    _link([objects[name] for name in PROBE_SOURCES], PROBE_LIBRARY)
-    build_front()
-    BUILD_INFO.write_text(json.dumps({'git_head': git_head(),
-                                      'library_sha256': hashlib.sha256(LIBRARY.read_bytes()).hexdigest()}) + '\n')
+    linked = [(_link([objects[name] for name in SOURCES], LIBRARY), LIBRARY),
+              (_link([objects[name] for name in PROBE_SOURCES], PROBE_LIBRARY), PROBE_LIBRARY)]
+    FRONT_LIBRARY.unlink(missing_ok=True)
+    for tmp, library in linked:
+        os.replace(tmp, library)
+    info = {'git_head': git_head(), 'library_sha256': file_sha256(LIBRARY)}
+    BUILD_INFO.write_text(json.dumps(info) + '\n')
+    front, target = build_front()
+    if front is None:
+        print(f'the torch front end is left out: {target}', file=sys.stderr)
+    else:
+        BUILD_INFO.write_text(json.dumps({**info, 'front_sha256': file_sha256(front), **target}) + '\n')
+        os.replace(front, FRONT_LIBRARY)
     return LIBRARY
 
 
