@@ -1,6 +1,7 @@
 """The front end's native calls against its Python route (which a tensor
-subclass takes): the same bits for every option, the caller's own output
-tensor back, the current stream, and the same errors."""
+subclass takes, and what else needs Python): the same bits for every option, the
+caller's own output tensor back, the current stream, and the same errors.  Every
+comparison first shows that its Python leg is one."""
 import pytest
 
 from redshift_amd import attention as A
@@ -19,8 +20,19 @@ def make(torch, dtype, tokens=5, position=700, seed=0):
 
 
 def python_route(t):
+    """t as a tensor subclass (nn.Parameter is none to the native calls)."""
     import torch
-    return torch.nn.Parameter(t, requires_grad=False)
+
+    class Subclass(torch.Tensor):
+        pass
+    return t.as_subclass(Subclass)
+
+
+def native(name, *args):
+    """The native call; None for what it does not take."""
+    front = A._FRONT or A._load_front()
+    assert front is not A._PythonRoute
+    return getattr(front, name)(*args)
 
 
 @pytest.mark.parametrize('dtype', ['float16', 'bfloat16'])
@@ -36,16 +48,40 @@ def test_attention_routes_agree(gpu, dtype, out, ws):
         kw['out'] = torch.zeros(q.shape, dtype=torch.float32 if 'float32' in out else q.dtype, device='cuda')
     elif out == 'float32':
         kw['out_dtype'] = torch.float32
-    native = A._load_front().attention(q, cache, 700, 1 / 16, kw.get('out'), kw.get('ws'), kw.get('out_dtype'))
-    assert native is not None and (native is kw['out'] if 'out' in kw else True)
-    native = native.clone()
-    other = A.attention(python_route(q), cache, 700, 1 / 16, **kw)
-    assert native.dtype == other.dtype and native.shape == other.shape and torch.equal(native, other)
-    # A strided query takes the Python route (a copy); so does an int scale.
+
+    def options():
+        fresh = dict(kw)
+        if 'out' in kw:
+            fresh['out'] = torch.full_like(kw['out'], float('nan'))
+        return fresh, (fresh.get('out'), fresh.get('ws'), fresh.get('out_dtype'))
+
+    fresh, rest = options()
+    want = native('attention', q, cache, 700, 1 / 16, *rest)
+    assert want is not None and (want is fresh['out'] if 'out' in kw else True)
+    assert native('attention', torch.nn.Parameter(q, requires_grad=False), cache, 700, 1 / 16, *rest) is not None
     wide = torch.zeros(5, 24, 512, dtype=q.dtype, device='cuda')
     wide[..., ::2] = q
-    assert A._load_front().attention(wide[..., ::2], cache, 700, 1 / 16, None, None, None) is None
-    assert torch.equal(A.attention(wide[..., ::2], cache, 700, 1 / 16, **kw), native)
+    for query in (python_route(q), wide[..., ::2]):
+        fresh, rest = options()
+        assert native('attention', query, cache, 700, 1 / 16, *rest) is None
+        got = A.attention(query, cache, 700, 1 / 16, **fresh)
+        assert got is fresh['out'] if 'out' in kw else type(got) is torch.Tensor
+        assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want)
+
+
+def test_what_only_python_takes(gpu):
+    """An integer scale, a subclass as output, workspace or cache tensor."""
+    torch = gpu
+    cache, q = make(torch, torch.float16)
+    ws = A.workspace(A.attention_workspace_bytes(24, 4, 256, 5, 700))
+    want = native('attention', q, cache, 700, 1.0, None, None, None)
+    out = python_route(torch.zeros_like(q))
+    for scale, o, w in ((1, None, None), (1.0, out, None), (1.0, None, python_route(ws))):
+        assert native('attention', q, cache, 700, scale, o, w, None) is None
+        assert torch.equal(A.attention(q, cache, 700, scale, out=o, ws=w).as_subclass(torch.Tensor), want)
+    cache.k = python_route(cache.k)
+    assert native('attention', q, cache, 700, 1.0, None, None, None) is None
+    assert torch.equal(A.attention(q, cache, 700, 1.0), want)
 
 
 @pytest.mark.parametrize('tokens,position', [(1, 0), (3, 40), (2, 700), (8, 700), (40, 700)])
@@ -56,15 +92,20 @@ def test_fused_routes_agree(gpu, tokens, position):
                                                                     (tokens, 4, 256), (256,), (256,))]
     side = torch.cuda.Stream()
     outs = []
-    for route in ('native', 'stream', 'python', 'unaligned'):
+    for route in ('native', 'stream', 'python', 'subclass key', 'unaligned'):
         cache, _ = make(torch, torch.float16, tokens, position)
         x = list(inputs)
         if route == 'python':
             x[0] = python_route(x[0])
+        if route == 'subclass key':
+            x[1] = python_route(x[1])
         if route == 'unaligned':   # 4 bytes off a 16-byte boundary: copied in Python
             buf = torch.zeros(x[1].numel() + 1, device='cuda')
             buf[1:] = x[1].reshape(-1)
             x[1] = buf[1:].view(x[1].shape)
+        assert (native('attention_fused', *x, cache, position, 1e-6, None, None) is None) == (
+            route in ('python', 'subclass key', 'unaligned'))
+        cache, _ = make(torch, torch.float16, tokens, position)   # as it was before that call
         torch.cuda.synchronize()
         with torch.cuda.stream(side if route == 'stream' else torch.cuda.current_stream()):
             outs.append(A.attention_fused(*x, cache, position, 1e-6))
@@ -88,6 +129,13 @@ def test_errors_are_the_python_ones(gpu):
         for query in (q, python_route(q)):
             with pytest.raises(kind, match=match):
                 A.attention(query, cache, **args)
+        rest = [args.get(n) for n in ('out', 'ws', 'out_dtype')]
+        assert native('attention', python_route(q), cache, args['position'], args['scale'], *rest) is None
+        if kind is RuntimeError:   # an error of the library: from either route
+            with pytest.raises(kind, match=match):
+                native('attention', q, cache, args['position'], args['scale'], *rest)
+        else:
+            assert native('attention', q, cache, args['position'], args['scale'], *rest) is None
     with pytest.raises(ValueError, match='q is torch.bfloat16'):
         A.attention(q.bfloat16(), cache, 700, 1 / 16)
     x = [torch.zeros(s, device='cuda') for s in ((2, 24, 512), (2, 4, 256), (2, 4, 256), (256,), (256,))]
