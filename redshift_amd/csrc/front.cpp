@@ -3,14 +3,16 @@
 // tensors, allocates the output and calls the C ABI.  An eager decode or
 // verification layer is two kernels of 7 to 19 us; checked and launched from
 // Python through ctypes it took the host 16-18 us (raw) and 31 us (a session's
-// layer), so the GPU waited for the host.  Of that the two launches
-// themselves are about 7 us.
+// layer), so the GPU waited for the host.  Of that the C call itself is about
+// 4 us for one launch and 8 for two.
 //
 // Every function returns None, before anything is enqueued, for a call that
-// it does not take (a tensor subclass, a tensor that needs a copy, a wrong
-// type, shape or device, a call off the GPU); attention.py then does the same
-// in Python, copies included, or raises its error.  An error of the library
-// is raised here, as redshift_amd.runtime.check raises it.
+// it does not take (a tensor subclass, which nn.Parameter is not here, a tensor
+// that needs a copy, a wrong type, shape or device, a call off the GPU);
+// attention.py then does the same in Python, copies included, or raises its
+// error.  No exception is thrown for a refusal, which would cost the call 2 us
+// (a strided query 20.4 against 18.2 us of host time, 19.4 in Python alone).  An
+// error of the library is raised here, as redshift_amd.runtime.check raises it.
 //
 // Tensors are read through their public metadata; nothing is kept between
 // calls but the library's function pointers.
@@ -21,223 +23,233 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <limits>
-#include <optional>
+#include <utility>
+
+#include "runtime.h"
 
 namespace {
 
-using Attention = int (*)(void *, const void *, const void *, const void *, int, int, int, int, int, int, int, int,
-                          float, void *, uint64_t, void *);
-using AttentionWorkspace = int (*)(uint64_t *, int, int, int, int, int);
-using Fused = int (*)(float *, void *, void *, const float *, const float *, const float *, const float *,
-                      const float *, int, int, int, float, void *, uint64_t, void *);
-using FusedWorkspace = int (*)(uint64_t *, int, int);
-using Error = const char *(*)();
-
-constexpr int kF16 = 1, kBF16 = 2, kF32 = 3;                       // include/runtime.h
 constexpr int kQHeads = 24, kKvHeads = 4, kHeadDim = 256;          // the fused model
 constexpr uint64_t kMinWorkspace = 256;
 
-Attention attention = nullptr;
-AttentionWorkspace attention_workspace = nullptr;
-Fused fused = nullptr;
-FusedWorkspace fused_workspace = nullptr;
-Error last_error = nullptr;
+decltype(&qv_attention) attention = nullptr;
+decltype(&qv_attention_workspace) attention_workspace = nullptr;
+decltype(&qv_attention_fused) fused = nullptr;
+decltype(&qv_attention_fused_workspace) fused_workspace = nullptr;
+decltype(&qv_error) last_error = nullptr;
 PyObject *get_device = nullptr, *get_stream = nullptr;
 PyObject *name_k, *name_v, *name_dtype, *name_kv_heads, *name_head_dim, *name_capacity;
 
 // A call this module does not take.
-struct NotTaken {};
-void require(bool condition) {
-    if (!condition) throw NotTaken{};
+PyObject *not_taken() {
+    PyErr_Clear();
+    Py_RETURN_NONE;
 }
 
+// The readers below return false for what the module does not take.
 // A plain torch tensor (subclasses go to Python).
-const at::Tensor &tensor(PyObject *o) {
-    require(THPVariable_CheckExact(o));
-    const at::Tensor &t = THPVariable_Unpack(o);
-    require(t.defined() && t.layout() == at::kStrided && t.has_storage());
-    return t;
+bool tensor(PyObject *o, const at::Tensor *&t) {
+    if (!THPVariable_CheckExact(o)) return false;
+    t = &THPVariable_Unpack(o);
+    return t->defined() && t->layout() == at::kStrided && t->has_storage();
 }
 
-int integer(PyObject *o) {
-    require(PyLong_CheckExact(o));
+bool integer(PyObject *o, int &value) {
+    if (!PyLong_CheckExact(o)) return false;
     int overflow = 0;
     const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
-    require(!overflow && v >= std::numeric_limits<int>::min() && v <= std::numeric_limits<int>::max());
-    return (int)v;
+    if (overflow || v < std::numeric_limits<int>::min() || v > std::numeric_limits<int>::max()) return false;
+    value = (int)v;
+    return true;
 }
 
-float real(PyObject *o) {
-    require(PyFloat_Check(o));
-    return (float)PyFloat_AS_DOUBLE(o);
+bool real(PyObject *o, float &value) {
+    if (!PyFloat_Check(o)) return false;
+    value = (float)PyFloat_AS_DOUBLE(o);
+    return true;
 }
 
 struct Ref {
-    PyObject *o;
+    PyObject *o = nullptr;
     ~Ref() { Py_XDECREF(o); }
 };
 
-// A PagedKV's fields.
+// A PagedKV's fields (its tensors held while the call runs).
 struct Cache {
     Ref k_ref, v_ref;
-    at::Tensor k, v;
-    at::ScalarType dtype;
-    int kv_heads, head_dim, capacity;
-    explicit Cache(PyObject *o)
-        : k_ref{PyObject_GetAttr(o, name_k)}, v_ref{PyObject_GetAttr(o, name_v)} {
-        require(k_ref.o && v_ref.o);
-        k = tensor(k_ref.o);
-        v = tensor(v_ref.o);
-        require(k.is_cuda() && v.device() == k.device());
+    const at::Tensor *k = nullptr, *v = nullptr;
+    at::ScalarType dtype = at::ScalarType::Undefined;
+    int kv_heads = 0, head_dim = 0, capacity = 0;
+
+    bool read(PyObject *o) {
+        k_ref.o = PyObject_GetAttr(o, name_k);
+        v_ref.o = k_ref.o ? PyObject_GetAttr(o, name_v) : nullptr;
+        if (!v_ref.o || !tensor(k_ref.o, k) || !tensor(v_ref.o, v)) return false;
+        if (!k->is_cuda() || v->device() != k->device()) return false;
         Ref d{PyObject_GetAttr(o, name_dtype)};
-        require(d.o && THPDtype_Check(d.o));
+        if (!d.o || !THPDtype_Check(d.o)) return false;
         dtype = reinterpret_cast<THPDtype *>(d.o)->scalar_type;
-        kv_heads = field(o, name_kv_heads);
-        head_dim = field(o, name_head_dim);
-        capacity = field(o, name_capacity);
+        return field(o, name_kv_heads, kv_heads) && field(o, name_head_dim, head_dim) &&
+               field(o, name_capacity, capacity);
     }
-    static int field(PyObject *o, PyObject *name) {
+    static bool field(PyObject *o, PyObject *name, int &value) {
         Ref f{PyObject_GetAttr(o, name)};
-        require(f.o);
-        return integer(f.o);
+        return f.o && integer(f.o, value);
     }
 };
 
 // torch's current stream, as torch.cuda.current_stream() gives it.
-void *current_stream() {
+bool current_stream(void *&stream) {
     Ref device{PyObject_CallNoArgs(get_device)};
-    require(device.o);
-    Ref stream{PyObject_CallOneArg(get_stream, device.o)};
-    require(stream.o);
-    void *s = PyLong_AsVoidPtr(stream.o);
-    require(!PyErr_Occurred());
-    return s;
+    Ref s{device.o ? PyObject_CallOneArg(get_stream, device.o) : nullptr};
+    if (!s.o) return false;
+    stream = PyLong_AsVoidPtr(s.o);
+    return !PyErr_Occurred();
 }
+
+// The call's allocations and launches run without the interpreter's lock, as
+// torch.empty and ctypes run them: an allocation may wait for the device.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 
 PyObject *raise_library_error() {
     const char *message = last_error();
-    Ref text{PyUnicode_DecodeUTF8(message, (Py_ssize_t)strlen(message), "replace")};
+    Ref text{PyUnicode_DecodeUTF8(message, (Py_ssize_t)std::strlen(message), "replace")};
     if (text.o) PyErr_SetObject(PyExc_RuntimeError, text.o);
     return nullptr;
 }
 
-// Runs `call`; None when it takes no such call.
-template <class Call>
-PyObject *taken(Call call) {
-    try {
-        return call();
-    } catch (...) {
-        PyErr_Clear();
-        Py_RETURN_NONE;
-    }
-}
-
-// The caller's workspace, or one of `bytes` on `like`'s device.
-at::Tensor workspace_of(PyObject *given, uint64_t bytes, const at::Tensor &like) {
-    if (given != Py_None) return tensor(given);
+// A workspace of `bytes` on `like`'s device.
+at::Tensor make_workspace(uint64_t bytes, const at::Tensor &like) {
     return at::empty({(int64_t)std::max(bytes, kMinWorkspace)}, like.options().dtype(at::kByte));
-}
-
-int code_of(at::ScalarType t) {
-    require(t == at::kHalf || t == at::kBFloat16);
-    return t == at::kHalf ? kF16 : kBF16;
 }
 
 // attention(q, cache, position, scale, out, ws, out_dtype)
 PyObject *py_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    return taken([&]() -> PyObject * {
-        require(n == 7 && attention);
-        const at::Tensor &q = tensor(args[0]);
-        const Cache cache(args[1]);
-        const int position = integer(args[2]);
-        const float scale = real(args[3]);
-        require(q.dim() == 3 && q.scalar_type() == cache.dtype && q.size(2) == cache.head_dim &&
-                q.device() == cache.k.device() && q.is_contiguous());
-        require(q.size(0) <= std::numeric_limits<int>::max() && q.size(1) <= std::numeric_limits<int>::max());
-        const int tokens = (int)q.size(0), q_heads = (int)q.size(1), dtype = code_of(cache.dtype);
-        at::Tensor out;
-        if (args[4] != Py_None) {
-            out = tensor(args[4]);
-            require(out.sizes() == q.sizes() && out.is_contiguous() && out.device() == q.device());
-        } else {
-            at::ScalarType t = cache.dtype;
-            if (args[6] != Py_None) {
-                require(THPDtype_Check(args[6]));
-                t = reinterpret_cast<THPDtype *>(args[6])->scalar_type;
-            }
-            require(t == cache.dtype || t == at::kFloat);
-            out = at::empty(q.sizes(), q.options().dtype(t));
+    constexpr int64_t kMost = std::numeric_limits<int>::max();
+    const at::Tensor *q = nullptr, *out = nullptr, *ws = nullptr;
+    Cache cache;
+    int position = 0;
+    float scale = 0.f;
+    if (n != 7 || !attention || !tensor(args[0], q) || !cache.read(args[1]) || !integer(args[2], position) ||
+        !real(args[3], scale))
+        return not_taken();
+    if (cache.dtype != at::kHalf && cache.dtype != at::kBFloat16) return not_taken();
+    if (q->dim() != 3 || q->scalar_type() != cache.dtype || q->size(2) != cache.head_dim ||
+        q->device() != cache.k->device() || !q->is_contiguous() || q->size(0) > kMost || q->size(1) > kMost)
+        return not_taken();
+    const int tokens = (int)q->size(0), q_heads = (int)q->size(1);
+    at::ScalarType out_type = cache.dtype;
+    if (args[4] != Py_None) {
+        if (!tensor(args[4], out) || out->sizes() != q->sizes() || !out->is_contiguous() ||
+            out->device() != q->device())
+            return not_taken();
+        out_type = out->scalar_type();
+    } else if (args[6] != Py_None) {
+        if (!THPDtype_Check(args[6])) return not_taken();
+        out_type = reinterpret_cast<THPDtype *>(args[6])->scalar_type;
+    }
+    if (out_type != cache.dtype && out_type != at::kFloat) return not_taken();
+    if (args[5] != Py_None && (!tensor(args[5], ws) || ws->device() != q->device())) return not_taken();
+    void *stream = nullptr;
+    if (!current_stream(stream)) return not_taken();
+    const int dtype = cache.dtype == at::kHalf ? QV_F16 : QV_BF16, out_code = out_type == at::kFloat ? QV_F32 : dtype;
+    int code = 0;
+    at::Tensor made;
+    try {
+        const void *qp = q->data_ptr(), *k = cache.k->data_ptr(), *v = cache.v->data_ptr();
+        void *o = out ? out->data_ptr() : nullptr, *w = ws ? ws->data_ptr() : nullptr;
+        uint64_t bytes = ws ? (uint64_t)ws->nbytes() : 0;
+        at::Tensor scratch;
+        Unlocked unlocked;
+        if (!out) {
+            made = at::empty(q->sizes(), q->options().dtype(out_type));
+            o = made.data_ptr();
         }
-        require(out.scalar_type() == cache.dtype || out.scalar_type() == at::kFloat);
-        uint64_t bytes = 0;
-        if (args[5] == Py_None && attention_workspace(&bytes, q_heads, cache.kv_heads, cache.head_dim, tokens, position))
-            return raise_library_error();
-        const at::Tensor ws = workspace_of(args[5], bytes, q);
-        require(ws.device() == q.device());
-        void *stream = current_stream();
-        const int out_code = out.scalar_type() == at::kFloat ? kF32 : dtype;
-        void *o = out.data_ptr(), *w = ws.data_ptr();
-        const void *qp = q.data_ptr(), *k = cache.k.data_ptr(), *v = cache.v.data_ptr();
-        const uint64_t ws_bytes = (uint64_t)ws.nbytes();
-        int code;
-        Py_BEGIN_ALLOW_THREADS
-        code = attention(o, qp, k, v, dtype, out_code, q_heads, cache.kv_heads, cache.head_dim, tokens, position,
-                         cache.capacity, scale, w, ws_bytes, stream);
-        Py_END_ALLOW_THREADS
-        if (code) return raise_library_error();
-        if (args[4] != Py_None) return Py_NewRef(args[4]);
-        return THPVariable_Wrap(std::move(out));
-    });
+        if (!ws) {
+            code = attention_workspace(&bytes, q_heads, cache.kv_heads, cache.head_dim, tokens, position);
+            if (!code) {
+                scratch = make_workspace(bytes, *q);
+                w = scratch.data_ptr();
+                bytes = (uint64_t)scratch.nbytes();
+            }
+        }
+        if (!code)
+            code = attention(o, qp, k, v, dtype, out_code, q_heads, cache.kv_heads, cache.head_dim, tokens, position,
+                             cache.capacity, scale, w, bytes, stream);
+    } catch (...) {
+        return not_taken();   // nothing was launched (an allocation failed): Python raises it
+    }
+    if (code) return raise_library_error();
+    return out ? Py_NewRef(args[4]) : THPVariable_Wrap(std::move(made));
 }
 
 // attention_fused(q_gate, key, value, q_norm, k_norm, cache, position, epsilon, out, ws)
 PyObject *py_attention_fused(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    return taken([&]() -> PyObject * {
-        require(n == 10 && fused);
-        const Cache cache(args[5]);
-        const int position = integer(args[6]);
-        const float epsilon = real(args[7]);
-        require(cache.dtype == at::kHalf && cache.kv_heads == kKvHeads && cache.head_dim == kHeadDim);
-        const at::Tensor &q_gate = tensor(args[0]);
-        require(q_gate.dim() >= 1 && q_gate.size(0) <= std::numeric_limits<int>::max());
-        const int64_t batch = q_gate.size(0);
-        const int64_t numel[5] = {batch * kQHeads * 2 * kHeadDim, batch * kKvHeads * kHeadDim,
-                                  batch * kKvHeads * kHeadDim, kHeadDim, kHeadDim};
+    Cache cache;
+    int position = 0;
+    float epsilon = 0.f;
+    if (n != 10 || !fused || !cache.read(args[5]) || !integer(args[6], position) || !real(args[7], epsilon))
+        return not_taken();
+    if (cache.dtype != at::kHalf || cache.kv_heads != kKvHeads || cache.head_dim != kHeadDim) return not_taken();
+    const at::Tensor *t[5] = {}, *out = nullptr, *ws = nullptr;
+    for (int i = 0; i < 5; ++i)
+        if (!tensor(args[i], t[i])) return not_taken();
+    if (t[0]->dim() < 1 || t[0]->size(0) > std::numeric_limits<int>::max()) return not_taken();
+    const int64_t batch = t[0]->size(0);
+    const int64_t numel[5] = {batch * kQHeads * 2 * kHeadDim, batch * kKvHeads * kHeadDim,
+                              batch * kKvHeads * kHeadDim, kHeadDim, kHeadDim};
+    for (int i = 0; i < 5; ++i)
+        if (t[i]->scalar_type() != at::kFloat || t[i]->numel() != numel[i] || t[i]->device() != cache.k->device() ||
+            !t[i]->is_contiguous())
+            return not_taken();
+    if (args[8] != Py_None &&
+        (!tensor(args[8], out) || out->scalar_type() != at::kFloat || out->numel() != batch * kQHeads * kHeadDim ||
+         !out->is_contiguous() || out->device() != cache.k->device()))
+        return not_taken();
+    if (args[9] != Py_None && (!tensor(args[9], ws) || ws->device() != cache.k->device())) return not_taken();
+    void *stream = nullptr;
+    if (!current_stream(stream)) return not_taken();
+    int code = 0;
+    at::Tensor made;
+    try {
         const float *in[5];
         for (int i = 0; i < 5; ++i) {
-            const at::Tensor &t = tensor(args[i]);
-            require(t.scalar_type() == at::kFloat && t.numel() == numel[i] && t.device() == cache.k.device() &&
-                    t.is_contiguous());
-            in[i] = static_cast<const float *>(t.data_ptr());
-            require(reinterpret_cast<uintptr_t>(in[i]) % 16 == 0);
+            in[i] = static_cast<const float *>(t[i]->data_ptr());
+            if (reinterpret_cast<uintptr_t>(in[i]) % 16) return not_taken();
         }
-        at::Tensor out;
-        if (args[8] != Py_None) {
-            out = tensor(args[8]);
-            require(out.scalar_type() == at::kFloat && out.numel() == batch * kQHeads * kHeadDim &&
-                    out.is_contiguous() && out.device() == cache.k.device());
-        } else {
-            out = at::empty({batch, kQHeads, kHeadDim}, q_gate.options());
+        void *k = cache.k->data_ptr(), *v = cache.v->data_ptr();
+        float *o = out ? static_cast<float *>(out->data_ptr()) : nullptr;
+        void *w = ws ? ws->data_ptr() : nullptr;
+        uint64_t bytes = ws ? (uint64_t)ws->nbytes() : 0;
+        at::Tensor scratch;
+        Unlocked unlocked;
+        if (!out) {
+            made = at::empty({batch, kQHeads, kHeadDim}, t[0]->options());
+            o = static_cast<float *>(made.data_ptr());
         }
-        uint64_t bytes = 0;
-        if (args[9] == Py_None && fused_workspace(&bytes, (int)batch, position)) return raise_library_error();
-        const at::Tensor ws = workspace_of(args[9], bytes, q_gate);
-        require(ws.device() == cache.k.device());
-        void *stream = current_stream();
-        float *o = static_cast<float *>(out.data_ptr());
-        void *k = cache.k.data_ptr(), *v = cache.v.data_ptr(), *w = ws.data_ptr();
-        const uint64_t ws_bytes = (uint64_t)ws.nbytes();
-        int code;
-        Py_BEGIN_ALLOW_THREADS
-        code = fused(o, k, v, in[0], in[1], in[2], in[3], in[4], (int)batch, position, cache.capacity, epsilon, w,
-                     ws_bytes, stream);
-        Py_END_ALLOW_THREADS
-        if (code) return raise_library_error();
-        if (args[8] != Py_None) return Py_NewRef(args[8]);
-        return THPVariable_Wrap(std::move(out));
-    });
+        if (!ws) {
+            code = fused_workspace(&bytes, (int)batch, position);
+            if (!code) {
+                scratch = make_workspace(bytes, *t[0]);
+                w = scratch.data_ptr();
+                bytes = (uint64_t)scratch.nbytes();
+            }
+        }
+        if (!code)
+            code = fused(o, k, v, in[0], in[1], in[2], in[3], in[4], (int)batch, position, cache.capacity, epsilon, w,
+                         bytes, stream);
+    } catch (...) {
+        return not_taken();   // nothing was launched (an allocation failed): Python raises it
+    }
+    if (code) return raise_library_error();
+    return out ? Py_NewRef(args[8]) : THPVariable_Wrap(std::move(made));
 }
 
 // bind(qv_attention, qv_attention_workspace, qv_attention_fused,
@@ -256,11 +268,11 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
             return nullptr;
         }
     }
-    attention = reinterpret_cast<Attention>(f[0]);
-    attention_workspace = reinterpret_cast<AttentionWorkspace>(f[1]);
-    fused = reinterpret_cast<Fused>(f[2]);
-    fused_workspace = reinterpret_cast<FusedWorkspace>(f[3]);
-    last_error = reinterpret_cast<Error>(f[4]);
+    attention = reinterpret_cast<decltype(attention)>(f[0]);
+    attention_workspace = reinterpret_cast<decltype(attention_workspace)>(f[1]);
+    fused = reinterpret_cast<decltype(fused)>(f[2]);
+    fused_workspace = reinterpret_cast<decltype(fused_workspace)>(f[3]);
+    last_error = reinterpret_cast<decltype(last_error)>(f[4]);
     Py_XSETREF(get_device, Py_NewRef(args[5]));
     Py_XSETREF(get_stream, Py_NewRef(args[6]));
     Py_RETURN_NONE;
