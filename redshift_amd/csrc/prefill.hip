@@ -380,9 +380,9 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
     // the change get weights within 2^-13 * ln 2 of each other.
     constexpr float kFoldMax = 4096.f;
     float sign = a.scale_sign, scale = a.scale_size, lazy = a.lazy;
-    // Scores that take a sign (or the whole scale) first do so where keys are
-    // masked: then on every page.
-    wave_first_limit = min(wave_first_limit, a.mask_from);
+    // Scores that take a sign (or the whole scale) do so beside the masks: then
+    // on every page, otherwise from the first page with a masked key.
+    int work_from = min(wave_first_limit, a.mask_from);
     float move_above[NT], neg_mu[NT];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
@@ -438,13 +438,17 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             const int key0 = (p0 + i) * 32;
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = s[tt][j >> 2][j & 3];
-            if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo)) {
+            if (key0 + 31 > work_from || (PK && key0 < key_lo)) {
                 keep_branch();
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int key = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
-                    x[j] *= sign;
-                    if (key > limit[tt] || (PK && key < key_lo)) x[j] = -INFINITY;
+                for (int j = 0; j < 8; ++j) x[j] *= sign;
+                if (key0 + 31 > wave_first_limit || (PK && key0 < key_lo)) {
+                    keep_branch();
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int key = key0 + 16 * (j >> 2) + 4 * g + (j & 3);
+                        if (key > limit[tt] || (PK && key < key_lo)) x[j] = -INFINITY;
+                    }
                 }
             }
             mx = __builtin_fmaxf(max3(x[0], x[1], x[2]), max3(x[3], x[4], x[5]));
@@ -483,7 +487,7 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
                     sign = a.scale_log2;
                     scale = 1.f;
                     lazy = kLazy;
-                    wave_first_limit = INT_MIN;
+                    work_from = INT_MIN;
 #pragma unroll
                     for (int t2 = 0; t2 < NT; ++t2) move_above[t2] = m[t2] + kLazy;
                 }
@@ -919,7 +923,8 @@ __device__ __forceinline__ void prefill_rows(const PrefillArgs &a, KV *kring, VT
             nl = max(0, (wg_keys + 31) / 32 - p0);
             nw = min(max((wave_keys + 31) / 32 - p0, 0), nl);
             limit[0] = a.position + row_token;
-            wave_first_limit = min(sign == a.scale_sign ? a.mask_from : INT_MIN, a.position + max(row0, 0) / a.group);
+            wave_first_limit = a.position + max(row0, 0) / a.group;
+            work_from = min(sign == a.scale_sign ? a.mask_from : INT_MIN, wave_first_limit);
             key_lo = a.position;
             prep_new_keys();
             s[0][0] = s[0][1] = f32x4{0.f, 0.f, 0.f, 0.f};
