@@ -1135,7 +1135,7 @@ void attention_prefill_bf16(PrefillArgs a) {
 //     work, but a round of workgroups that is not full is lost whole.  Taken
 //     for one round at most (1500 tokens of 32/8/128 at 0: 32.1, with pairs
 //     39.3).
-//   Pairs, four waves (216 VGPRs, 64 KiB of rings: two workgroups per CU): for
+//   Pairs, four waves (213 VGPRs, 64 KiB of rings: two workgroups per CU): for
 //     several rounds, the longest workgroups first and the CUs refilled as
 //     they end (2048 of 32/8/128 at 30,000: 999, 192-row workgroups 1581; 3000
 //     at 0: 83.1 and 107.8).  Two workgroups of a CU take about 5/4, and one
