@@ -30,12 +30,12 @@
 // the scale is folded into the exponents' multiply-add, its sign applied to
 // the scores first where it is not positive, so any finite scale (zero and
 // negative ones included) gives the softmax of the scaled scores as long as
-// these are finite in fp32 (kFoldMax below).  A page that
-// moves no row's max (nearly every page) needs neither the cross-lane row max
-// nor a rescaling factor: about 30 vector instructions and 8 exponentials per
-// page instead of 48 and 9 (bf16 2048 tokens at 6144: 330.3 -> 319.0 us; 3000
-// fp16 tokens of 32/8/128: 107.8 -> 100.9; the fused 2048-token chunk, bound
-// by its hi + lo products: 624.9 -> 619.2).  P multiplies V as one fp16 value.  On bf16 caches a
+// these are finite in fp32 (kFoldMax below).  A page that moves no row's max
+// (nearly every page) needs neither the cross-lane row max nor a rescaling
+// factor: about 30 vector instructions and 8 exponentials per page instead of
+// 48 and 9 (bf16 2048 tokens at 6144: 330.3 -> 319.0 us; 3000 fp16 tokens of
+// 32/8/128: 107.8 -> 100.9; the fused 2048-token chunk, bound by its hi + lo
+// products: 624.9 -> 619.2).  P multiplies V as one fp16 value.  On bf16 caches a
 // streaming pass (convert_v_pages) first writes the call's V pages as fp16
 // into the workspace, which is exact for every bf16 value from 2^-14 to
 // 65280 (the fp16 normal range), so bf16 runs one V product per fragment,
